@@ -58,11 +58,11 @@ constexpr size_t kInfinityCacheBytes = (size_t)256 << 20;  // MI355X's memory-si
 // prefetched ones included, before a block's first MFMA.
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint4 gload16(const void* p) {
-  return __builtin_bit_cast(uint4, *(const __attribute__((address_space(1))) u32x4_t*)p);
+__device__ __forceinline__ u32x4_t gload16(const void* p) {
+  return *(const __attribute__((address_space(1))) u32x4_t*)p;
 }
-__device__ __forceinline__ float4 gload16f(const void* p) {
-  return __builtin_bit_cast(float4, *(const __attribute__((address_space(1))) u32x4_t*)p);
+__device__ __forceinline__ f4v gload16f(const void* p) {
+  return *(const __attribute__((address_space(1))) f4v*)p;
 }
 __device__ __forceinline__ uint2 gload8(const void* p) {
   return __builtin_bit_cast(uint2, *(const __attribute__((address_space(1))) u32x2_t*)p);
@@ -157,8 +157,8 @@ __device__ __forceinline__ void k_ring(int k0, int nb, Load& load, Pin& pin, Mma
   }
 }
 
-__device__ __forceinline__ void pin4(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
-__device__ __forceinline__ void pin4(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+__device__ __forceinline__ void pin4(u32x4_t& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void pin4(f4v& v) { asm volatile("" : "+v"(v)); }
 
 template <int SW, int KB, bool kSmall, typename Frag, typename Load, typename Pin, typename Mma>
 __device__ __forceinline__ void k_loop(int first, int slice, Load&& load, Pin&& pin, Mma&& mma) {
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     const char* wr = weights + woff + ((size_t)(n0 / kBatchTile) * nkb * 64 + lane) * 4 * (P == kFp32 ? 4 : 2);
     const float* gr = reinterpret_cast<const float*>(weights + w_norm) + 4 * g;
     struct Frag {
-      float4 w[CT], gn, x[NT];
+      f4v w[CT], gn, x[NT];
     };
     auto load = [&](int k, Frag& f) {
 #pragma unroll
@@ -246,21 +246,21 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
           f.w[c] = gload16f(reinterpret_cast<const float*>(wr) + blk);
         } else {
           const uint2 h = gload8(reinterpret_cast<const uint16_t*>(wr) + blk);
-          f.w[c] = make_float4(half_to_float((unsigned short)(h.x & 0xffffu)), half_to_float((unsigned short)(h.x >> 16)),
-                               half_to_float((unsigned short)(h.y & 0xffffu)), half_to_float((unsigned short)(h.y >> 16)));
+          f.w[c] = f4v{half_to_float((unsigned short)(h.x & 0xffffu)), half_to_float((unsigned short)(h.x >> 16)),
+                       half_to_float((unsigned short)(h.y & 0xffffu)), half_to_float((unsigned short)(h.y >> 16))};
         }
       }
       // The norm vector holds `width` values (a multiple of 16): a group of 4 is all in or out.
-      f.gn = make_float4(0.f, 0.f, 0.f, 0.f);
+      f.gn = f4v{0.f, 0.f, 0.f, 0.f};
       if constexpr (kNorm)
         if (k + 4 * g < width) f.gn = gload16f(gr + k);
 #pragma unroll
-      for (int t = 0; t < NT; t++) f.x[t] = *reinterpret_cast<const float4*>(xr + ((size_t)t * nkb + k / 16) * 256);
+      for (int t = 0; t < NT; t++) f.x[t] = gload16f(xr + ((size_t)t * nkb + k / 16) * 256);
     };
     auto mma = [&](int i, const Frag& f) {
 #pragma unroll
       for (int t = 0; t < NT; t++) {
-        float4 x = f.x[t];
+        f4v x = f.x[t];
         if constexpr (kNorm) {
           ss[i][t] += x.x * x.x;
           ss[i][t] += x.y * x.y;
@@ -297,20 +297,20 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     const uint16_t* wr = reinterpret_cast<const uint16_t*>(weights + woff) + ((size_t)(n0 / kBatchTile) * nkb * 64 + lane) * 8;
     const uint16_t* gr = reinterpret_cast<const uint16_t*>(weights + w_norm) + 8 * g;
     struct Frag {
-      uint4 w[CT], gn;
-      float4 xlo[NT], xhi[NT];
+      u32x4_t w[CT], gn;
+      f4v xlo[NT], xhi[NT];
     };
     auto load = [&](int k, Frag& f) {
 #pragma unroll
       for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
-      f.gn = make_uint4(0u, 0u, 0u, 0u);
+      f.gn = u32x4_t{0u, 0u, 0u, 0u};
       if constexpr (kNorm)
         if (k + 8 * g < width) f.gn = gload16(gr + k);
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const float* p = xr + ((size_t)t * nkb + k / 32) * 512;
-        f.xlo[t] = *reinterpret_cast<const float4*>(p);
-        f.xhi[t] = *reinterpret_cast<const float4*>(p + 256);
+        f.xlo[t] = gload16f(p);
+        f.xhi[t] = gload16f(p + 256);
       }
     };
     auto mma = [&](int i, const Frag& f) {
@@ -367,13 +367,13 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     const uint16_t* xr = reinterpret_cast<const uint16_t*>(X) + ((size_t)t0 * nkb * 64 + lane) * 8;
     const uint16_t* wr = reinterpret_cast<const uint16_t*>(weights + woff) + ((size_t)(n0 / kBatchTile) * nkb * 64 + lane) * 8;
     struct Frag {
-      uint4 w[CT], x[NT];
+      u32x4_t w[CT], x[NT];
     };
     auto load = [&](int k, Frag& f) {
 #pragma unroll
       for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
 #pragma unroll
-      for (int t = 0; t < NT; t++) f.x[t] = *reinterpret_cast<const uint4*>(xr + ((size_t)t * nkb + k / 32) * 512);
+      for (int t = 0; t < NT; t++) f.x[t] = gload16(xr + ((size_t)t * nkb + k / 32) * 512);
     };
     auto mma = [&](int i, const Frag& f) {
 #pragma unroll
