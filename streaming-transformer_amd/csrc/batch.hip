@@ -98,6 +98,8 @@ Batch::Batch(const st_config& config, bool mixed, const st_tensor* tensors, size
   a.act = zeroed(act_, (size_t)streams_p_ * a.ffn_p);
   a.q = zeroed(q_, (size_t)streams_p_ * a.width);
   a.score = zeroed(score_, (size_t)streams_);
+  a.rope = reinterpret_cast<float2*>(zeroed(step_rope_, (size_t)streams_p_ * dim_));
+  a.slot = reinterpret_cast<int*>(zeroed(step_slot_, (size_t)streams_p_));
   host_in_.alloc((size_t)streams_p_ * a.features_p * 4);
   std::memset(host_in_.ptr, 0, (size_t)streams_p_ * a.features_p * 4);
   host_out_.alloc((size_t)streams_ * 4);
@@ -131,16 +133,29 @@ int Batch::group_tiles(int cols, int max_tiles) const {
 }
 
 template <int P, int E, bool kNorm, int CT, int SW>
-void Batch::project(const void* X, int ld, uint32_t woff, int N, uint32_t norm, int layer, int max_tiles) {
+void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer,
+                    int max_tiles) {
   const int cols = N / (kBatchTile * CT);
   const int nt = group_tiles(cols, max_tiles);
   const dim3 grid(cols, streams_p_ / kBatchTile / nt), block(64 * kSlices / SW);
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream_, dargs_, args_.weights, X, woff, N, ld, c_.width, norm, layer);
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream_, args_.weights, X, out, dargs_, woff, ld, norm, c_.width, streams_,
+                       out_ld, layer);
   };
-  if (nt == 4) go(batch_proj<P, E, kNorm, 4, CT, SW>);
-  else if (nt == 2) go(batch_proj<P, E, kNorm, 2, CT, SW>);
-  else go(batch_proj<P, E, kNorm, 1, CT, SW>);
+  // Blocks in flight per wave (k_ring): four where a slice holds a multiple of four and the
+  // workgroup has at most two tiles, else two.
+  constexpr int kb = P == kFp32 || (P == kMixed && E == kEpInput) ? 16 : 32;
+  const bool deep = ld / kSlices / kb % 4 == 0;
+  auto ring = [&](auto NT) {
+    constexpr int nt_ = decltype(NT)::value;
+    if constexpr (SW == 1 && nt_ * CT <= 2) {
+      if (deep) return go(batch_proj<P, E, kNorm, nt_, CT, SW, 4>);
+    }
+    go(batch_proj<P, E, kNorm, nt_, CT, SW, 2>);
+  };
+  if (nt == 4) ring(std::integral_constant<int, 4>{});
+  else if (nt == 2) ring(std::integral_constant<int, 2>{});
+  else ring(std::integral_constant<int, 1>{});
 }
 
 // Workgroup shapes per projection. Every shape computes the same fixed slice tree, so the
@@ -174,13 +189,13 @@ void Batch::launch_sequence() {
     if constexpr (!kFold)
       hipLaunchKernelGGL(batch_norm_mixed, dim3(streams_p_), dim3(256), 0, stream_, dargs_, w_norm);
   };
-  project<P, kEpInput, false, 1, 1>(a.in, a.features_p, a.w_input, d, 0u, 0);
+  project<P, kEpInput, false, 1, 1>(a.in, a.features_p, a.x, a.width_p, a.w_input, d, 0u, 0);
   for (int l = 0; l < c_.layers; l++) {
     const LayerWeights& w = a.layer[l];
     norm(w.norm1);
     if (wide && wide_qkv_)
-      project<P, kEpQkv, kFold, 2, 2>(nx, a.width_p, w.qkv, 3 * d, w.norm1, l, huge ? 1 : kGroupTiles);
-    else project<P, kEpQkv, kFold, 1, 1>(nx, a.width_p, w.qkv, 3 * d, w.norm1, l);
+      project<P, kEpQkv, kFold, 2, 2>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l, huge ? 1 : kGroupTiles);
+    else project<P, kEpQkv, kFold, 1, 1>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
     {
       const dim3 grid(streams_ * c_.heads), block(kAttnThreads);
       const size_t lds = (size_t)c_.window * 4;
@@ -198,14 +213,14 @@ void Batch::launch_sequence() {
       if (kv_nt) attend(std::true_type{});
       else attend(std::false_type{});
     }
-    if (narrow) project<P, kEpOut, false, 2, 1>(a.attn, a.width_p, w.out, d, 0u, l);
-    else project<P, kEpOut, false, 1, 1>(a.attn, a.width_p, w.out, d, 0u, l);
+    if (narrow) project<P, kEpOut, false, 2, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
+    else project<P, kEpOut, false, 1, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
     norm(w.norm2);
-    if (huge && (2 * F / kBatchTile) % 4 == 0) project<P, kEpGateUp, kFold, 4, 1>(nx, a.width_p, w.gateup, 2 * F, w.norm2, l);
-    else if (wide && wide_gateup_) project<P, kEpGateUp, kFold, 2, 2>(nx, a.width_p, w.gateup, 2 * F, w.norm2, l);
-    else project<P, kEpGateUp, kFold, 1, 1>(nx, a.width_p, w.gateup, 2 * F, w.norm2, l);
-    if (narrow) project<P, kEpDown, false, 2, 1>(a.act, a.ffn_p, w.down, d, 0u, l);
-    else project<P, kEpDown, false, 1, 1>(a.act, a.ffn_p, w.down, d, 0u, l);
+    if (huge && (2 * F / kBatchTile) % 4 == 0) project<P, kEpGateUp, kFold, 4, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+    else if (wide && wide_gateup_) project<P, kEpGateUp, kFold, 2, 2>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+    else project<P, kEpGateUp, kFold, 1, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+    if (narrow) project<P, kEpDown, false, 2, 1>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
+    else project<P, kEpDown, false, 1, 1>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
   }
   hipLaunchKernelGGL(batch_final<P>, dim3(streams_), dim3(64), 0, stream_, dargs_);
   HIP_CHECK(hipGetLastError());

@@ -44,7 +44,8 @@ class Batch : public BatchBase {
   }
   template <int P> void launch_sequence();
   template <int P, int E, bool kNorm, int CT, int SW>
-  void project(const void* X, int ld, uint32_t woff, int N, uint32_t norm, int layer, int max_tiles = kGroupTiles);
+  void project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer,
+               int max_tiles = kGroupTiles);
   int group_tiles(int cols, int max_tiles) const;
   void stage_events(const float* inputs, float* block) const;
   bool wide_qkv_ = false, wide_gateup_ = false;  // two column tiles per workgroup
@@ -61,7 +62,8 @@ class Batch : public BatchBase {
   StreamHandle stream_;
   GraphHandle graph_;
   GraphExecHandle graph_exec_;
-  DeviceBuffer weights_, keys_, values_, hidden_, position_, in_, x_, xn_, attn_, act_, q_, score_, rope_, args_dev_;
+  DeviceBuffer weights_, keys_, values_, hidden_, position_, in_, x_, xn_, attn_, act_, q_, score_, rope_, step_rope_, step_slot_,
+      args_dev_;
   PinnedBuffer host_in_, host_out_;
   StepArgs offsets_{};  // weight arena offsets (shared layout with the single-stream runtime)
   BatchArgs args_{};

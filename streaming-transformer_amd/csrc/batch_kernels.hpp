@@ -47,6 +47,8 @@ struct BatchArgs {
   float* act;                      // SwiGLU output (FP16 in mixed mode; ffn_p)
   float* q;                        // [Bp][width] rotated queries
   float* score;                    // [B]
+  float2* rope;                    // [Bp][dim / 2] cos, sin of this step's position (batch_proj, kEpInput)
+  int* slot;                       // [Bp] ring slot of this step's position
 };
 
 constexpr int kSlices = 8;       // K-slices of a projection, K / 8 columns each
@@ -66,6 +68,12 @@ __device__ __forceinline__ f4v gload16f(const void* p) {
 }
 __device__ __forceinline__ uint2 gload8(const void* p) {
   return __builtin_bit_cast(uint2, *(const __attribute__((address_space(1))) u32x2_t*)p);
+}
+
+// Any pointer read from the arguments block, in the global address space.
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* in_global(T* p) {
+  return (__attribute__((address_space(1))) T*)p;
 }
 
 // Activation layouts. The projections' operands (in, x, xn, attn, act) are stored the way the
@@ -122,60 +130,55 @@ __device__ __forceinline__ void split3(const float (&x)[8], unsigned (&ph)[4], u
   }
 }
 
-// The K loop of one wave over its SW slices, from slice `first`, in blocks of KB columns.
-// SW = 1: a ring of R fragments, unrolled so that no fragment is copied (a copy would wait for
-// its loads): block j + R is loaded into the fragment of block j as soon as block j's MFMAs are
-// issued, so R blocks are in flight while one computes. R = 4 for workgroups of at most two
+// The K loop of one wave over its SW slices, from slice `first`, in blocks of KB columns: a ring
+// of R steps (a step is one block of each slice), unrolled so that no fragment is copied: step
+// j + R is loaded into the fragments of step j as soon as step j's MFMAs are issued, so R steps
+// are in flight while one computes. The host picks R = 4 for one-slice waves of at most two
 // tiles when the slice holds a multiple of 4 blocks (it always holds an even number), else 2.
-// Two kinds of empty asm statement hold the schedule: one after each prefetch (the compiler
-// would otherwise see that the loads only feed the next round and move them next to their
-// use), and `pin`, which passes a fragment's registers through an asm right before its MFMAs
-// (the compiler would otherwise hoist the operand arithmetic of every fragment to the top of
-// the round, which waits for all loads in flight). Either way every block would wait a full
-// memory round trip. SW = 2: each step loads one block of each of the two slices, then runs
-// both. Every form issues a slice's MFMAs in block order.
-template <int R, int KB, typename Frag, typename Load, typename Pin, typename Mma>
-__device__ __forceinline__ void k_ring(int k0, int nb, Load& load, Pin& pin, Mma& mma) {
-  Frag f[R];
+// Three things hold the schedule: an empty asm after each prefetch (the compiler would otherwise
+// see that the loads only feed the next round and move them next to their use); `pin`, which
+// passes a fragment's registers through an asm right before its MFMAs (the compiler would
+// otherwise hoist the operand arithmetic of every fragment to the top of the round, which waits
+// for all loads in flight); and that the fragments are whole 4-register vectors in the pins too
+// (pinned as scalars, the loop carried a register copy per element, which waited for every
+// load at the end of each round: Large with bfloat16 weights at 32 streams 645 -> 595 us per step).
+// `early` runs once, when the first R steps' loads are in flight: the epilogue's own operands
+// are fetched there, so that their round trips overlap the loop's. Every form issues a slice's
+// MFMAs in block order.
+template <int R, int SW, int KB, typename Frag, typename Load, typename Pin, typename Mma, typename Early>
+__device__ __forceinline__ void k_ring(int first, int slice, Load&& load, Pin&& pin, Mma&& mma, Early&& early) {
+  const int nb = slice / KB;
+  Frag f[R][SW];
 #pragma unroll
-  for (int r = 0; r < R; r++) load(k0 + r * KB, f[r]);
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int i = 0; i < SW; i++) load((first + i) * slice + r * KB, f[r][i]);
   asm volatile("" ::: "memory");
+  early();
   int j = 0;
   for (; j + R < nb; j += R) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      pin(f[r]);
-      mma(0, f[r]);
-      load(k0 + (j + R + r) * KB, f[r]);
+#pragma unroll
+      for (int i = 0; i < SW; i++) {
+        pin(f[r][i]);
+        mma(i, f[r][i]);
+        load((first + i) * slice + (j + R + r) * KB, f[r][i]);
+      }
       asm volatile("" ::: "memory");
     }
   }
 #pragma unroll
-  for (int r = 0; r < R; r++) {
-    pin(f[r]);
-    mma(0, f[r]);
-  }
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int i = 0; i < SW; i++) {
+      pin(f[r][i]);
+      mma(i, f[r][i]);
+    }
 }
 
 __device__ __forceinline__ void pin4(u32x4_t& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin4(f4v& v) { asm volatile("" : "+v"(v)); }
-
-template <int SW, int KB, bool kSmall, typename Frag, typename Load, typename Pin, typename Mma>
-__device__ __forceinline__ void k_loop(int first, int slice, Load&& load, Pin&& pin, Mma&& mma) {
-  if constexpr (SW == 1) {
-    const int k0 = first * slice, nb = slice / KB;
-    if (kSmall && nb % 4 == 0) k_ring<4, KB, Frag>(k0, nb, load, pin, mma);
-    else k_ring<2, KB, Frag>(k0, nb, load, pin, mma);
-  } else {
-    for (int kk = 0; kk < slice; kk += KB) {
-      Frag f[SW];
-#pragma unroll
-      for (int i = 0; i < SW; i++) load((first + i) * slice + kk, f[i]);
-#pragma unroll
-      for (int i = 0; i < SW; i++) mma(i, f[i]);
-    }
-  }
-}
 
 // One projection Y = X . W^T over the batch, with its phase's epilogue. Workgroup: CT column
 // tiles of 16 outputs and NT batch tiles of 16 streams. K is cut into 8 slices; each wave
@@ -187,9 +190,7 @@ __device__ __forceinline__ void k_loop(int first, int slice, Load&& load, Pin&& 
 // the loops have no branches. X and W are in the tiled operand layout (act_index and the tiled
 // arena): one 16 x KB block of either is 64 lanes' contiguous 16-byte pieces in lane order.
 // X is the padded buffer of K columns; W the N x K matrix at offset `woff` of the arena
-// `weights`. What the K loop's first loads need (the arena, X, the shape) comes in the kernel
-// arguments, not from the arguments block, whose read would add a memory round trip before
-// them.
+// `weights`; `out` the phase's output buffer (row length out_ld): x, or the SwiGLU output.
 // FP32 weights: v_mfma_f32_16x16x4_f32, k block of 16; lane l supplies A[l % 16][l / 16] and
 // B[l / 16][l % 16], register r of lane l holds D[4 (l / 16) + r][l % 16]; the four MFMA
 // steps use k = kb + 4 (l / 16) + c for step c, the same index for A and B.
@@ -201,12 +202,19 @@ __device__ __forceinline__ void k_loop(int first, int slice, Load&& load, Pin&& 
 // (src/cuda/Primitives.cuh:122-135). The waves feed x * g to the MFMAs, accumulate the row's
 // sum of squares from the same loads, and the epilogue scales the row by
 // 1 / sqrt(sum / d + eps).
-template <int P, int E, bool kNorm, int NT, int CT, int SW>
-__global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs* __restrict__ ap,
-                                                               const char* __restrict__ weights,
-                                                               const void* __restrict__ X, uint32_t woff, int N,
-                                                               int K, int width, uint32_t w_norm, int layer) {
-  constexpr int kWaves = kSlices / SW;
+//
+// Everything a kernel needs before its first load comes in the kernel arguments (the first 16
+// dwords are preloaded into SGPRs). What only the epilogue needs (the residual, the RoPE table,
+// the ring geometry) is fetched while the K loop's first loads are in flight: read after the
+// loop, each of those was a dependent memory round trip on a kernel of 3-5 us (Main with
+// bfloat16 weights at 16 streams 195 -> 188 us per step, Large at 32 streams 595 -> 576 us).
+template <int P, int E, bool kNorm, int NT, int CT, int SW, int R>
+__global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __restrict__ weights,
+                                                               const void* __restrict__ X, void* out,
+                                                               const BatchArgs* __restrict__ ap, uint32_t woff, int K,
+                                                               uint32_t w_norm, int width, int streams, int out_ld,
+                                                               int layer) {
+  constexpr int kWaves = kSlices / SW, kBlock = 64 * kWaves;
   const BatchArgs& a = *ap;
   __shared__ float red[kWaves][NT][CT][16][17];
   __shared__ float sq[kWaves][NT][16];
@@ -216,6 +224,86 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
   const int r16 = lane & 15, g = lane >> 4;
   const int slice = K / kSlices;
   const int first = wave * SW;  // the wave's first slice
+
+  // Epilogue units of this thread: a column, or the column pair of a RoPE or gate-up pair, of
+  // one stream. Unit u of the workgroup's tiles is, for the phases that write an activation
+  // buffer, in the buffer's own order (four columns of a row, then the 16 rows), so that a wave
+  // stores (and loads the residual as) contiguous 256-byte runs; for QKV, whose outputs are
+  // row-major, a row's pairs are consecutive.
+  constexpr int unit = (E == kEpQkv || E == kEpGateUp) ? 2 : 1;
+  constexpr int per_row = kBatchTile * CT / unit;
+  constexpr int kUnits = NT * kBatchTile * per_row;
+  constexpr int kOwn = (kUnits + kBlock - 1) / kBlock;
+  struct Unit {
+    int t, row, cc;  // batch tile, row in it, first column in the workgroup's
+  };
+  auto unit_of = [&](int u) {
+    int o = (int)threadIdx.x + u * kBlock;
+    if (kUnits % kBlock != 0 && o >= kUnits) o = kUnits - 1;
+    if constexpr (E == kEpQkv) return Unit{o / (kBatchTile * per_row), (o / per_row) % kBatchTile, (o % per_row) * unit};
+    else return Unit{o / (kBatchTile * per_row), (o >> 2) % kBatchTile, ((o / 64) % (per_row / 4) * 4 + (o & 3)) * unit};
+  };
+  auto owned = [&](int u) { return kUnits % kBlock == 0 || (int)threadIdx.x + u * kBlock < kUnits; };
+
+  // Epilogue operands, fetched while the K loop's first loads are in flight. No branch around
+  // the loads: threads without a unit load the last unit's operands, and rows past the last
+  // stream are padding inside the buffers.
+  float res[kOwn];           // OUT, down: the residual x
+  v2f cs[kOwn];              // QKV: RoPE cos and sin of the pair
+  int slot[kOwn];            // QKV: the stream's ring slot
+  float epsilon = 0.f;
+  float *hidden = nullptr, *qkv_q = nullptr, *qkv_k = nullptr, *qkv_v = nullptr;
+  int layers = 0, dim = 1, heads = 1, window = 1;
+  auto early = [&] {
+    if constexpr (E == kEpInput) {
+      // This step's RoPE table and ring slots (src/cuda/Primitives.cuh:148-166), once per step
+      // instead of once per layer and unit: the workgroups of a batch tile group share its rows.
+      const int half = a.dim / 2, rows = NT * kBatchTile;
+      for (int i = (int)(blockIdx.x * kBlock + threadIdx.x); i < rows * half; i += (int)gridDim.x * kBlock) {
+        const int b = t0 * kBatchTile + i / half, j = i % half;
+        if (b >= streams) break;
+        const unsigned long long pos = a.position[b];
+        const float angle = (float)pos * a.rope_freq[j];
+        a.rope[(size_t)b * half + j] = make_float2(cosf(angle), sinf(angle));
+        if (j == 0) a.slot[b] = (int)(pos % (unsigned long long)a.window);
+      }
+    } else if constexpr (E == kEpQkv) {
+      epsilon = a.epsilon;
+      qkv_q = a.q;
+      qkv_k = reinterpret_cast<float*>(a.keys);
+      qkv_v = reinterpret_cast<float*>(a.values);
+      dim = a.dim;
+      heads = a.heads;
+      window = a.window;
+      const float2* rope = a.rope;
+      const int* slots = a.slot;
+      asm volatile("" ::"s"(epsilon), "s"(qkv_q), "s"(qkv_k), "s"(qkv_v), "s"(dim), "s"(heads), "s"(window), "s"(rope),
+                   "s"(slots), "s"(layer));
+#pragma unroll
+      for (int u = 0; u < kOwn; u++) {
+        const Unit o = unit_of(u);
+        const int b = (t0 + o.t) * kBatchTile + o.row;
+        cs[u] = __builtin_bit_cast(v2f, gload8(rope + (size_t)b * (dim / 2) + (n0 + o.cc) % dim / 2));
+        slot[u] = in_global(slots)[b];
+      }
+    } else if constexpr (E == kEpGateUp) {
+      if constexpr (kNorm) {
+        epsilon = a.epsilon;
+        asm volatile("" ::"s"(epsilon));
+      }
+    } else {
+      if constexpr (E == kEpDown) {
+        hidden = a.hidden;
+        layers = a.layers;
+        asm volatile("" ::"s"(hidden), "s"(layers), "s"(layer));
+      }
+#pragma unroll
+      for (int u = 0; u < kOwn; u++) {
+        const Unit o = unit_of(u);
+        res[u] = reinterpret_cast<const float*>(out)[act_index<P>((t0 + o.t) * kBatchTile + o.row, n0 + o.cc, out_ld)];
+      }
+    }
+  };
   f4v acc[SW][NT][CT];
   float ss[SW][NT];
 #pragma unroll
@@ -227,6 +315,10 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
       for (int c = 0; c < CT; c++) acc[i][t][c] = f4v{0.f, 0.f, 0.f, 0.f};
     }
   static_assert(!(kNorm && P == kMixed), "mixed mode materializes its norms");
+  // Index of the norm weights of columns k .. k + n - 1. The vector holds `width` values (a
+  // multiple of 16); padding columns, whose x is zero, take its last ones, so that the load has
+  // no branch around it (one in the K loop's rounds drained every load in flight).
+  auto norm_at = [&](int k, int n) { return k + n <= width ? k : width - n; };
   if constexpr (P == kFp32 || (P == kMixed && E == kEpInput)) {
     // FP32 MFMA. Mixed mode takes this path for the input projection only: its operand is
     // the raw FP32 event, and its FP16 weights widen exactly.
@@ -234,7 +326,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     const int nkb = K / 16;
     const float* xr = reinterpret_cast<const float*>(X) + ((size_t)t0 * nkb * 64 + lane) * 4;
     const char* wr = weights + woff + ((size_t)(n0 / kBatchTile) * nkb * 64 + lane) * 4 * (P == kFp32 ? 4 : 2);
-    const float* gr = reinterpret_cast<const float*>(weights + w_norm) + 4 * g;
+    const float* gr = reinterpret_cast<const float*>(weights + w_norm);
     struct Frag {
       f4v w[CT], gn, x[NT];
     };
@@ -250,10 +342,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
                        half_to_float((unsigned short)(h.y & 0xffffu)), half_to_float((unsigned short)(h.y >> 16))};
         }
       }
-      // The norm vector holds `width` values (a multiple of 16): a group of 4 is all in or out.
-      f.gn = f4v{0.f, 0.f, 0.f, 0.f};
-      if constexpr (kNorm)
-        if (k + 4 * g < width) f.gn = gload16f(gr + k);
+      if constexpr (kNorm) f.gn = gload16f(gr + norm_at(k + 4 * g, 4));
 #pragma unroll
       for (int t = 0; t < NT; t++) f.x[t] = gload16f(xr + ((size_t)t * nkb + k / 16) * 256);
     };
@@ -288,14 +377,14 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
       for (int t = 0; t < NT; t++) pin4(f.x[t]);
       if constexpr (kNorm) pin4(f.gn);
     };
-    k_loop<SW, 16, NT * CT <= 2, Frag>(first, slice, load, pin, mma);
+    k_ring<R, SW, 16, Frag>(first, slice, load, pin, mma, early);
   } else if constexpr (P == kBf16w) {
     // Tiled operands: weight block (tile, k / 32) holds 64 lanes x 8 values, activation block
     // two planes of 64 lanes x 4 floats.
     const int nkb = K / 32;
     const float* xr = reinterpret_cast<const float*>(X) + ((size_t)t0 * nkb * 128 + lane) * 4;
     const uint16_t* wr = reinterpret_cast<const uint16_t*>(weights + woff) + ((size_t)(n0 / kBatchTile) * nkb * 64 + lane) * 8;
-    const uint16_t* gr = reinterpret_cast<const uint16_t*>(weights + w_norm) + 8 * g;
+    const uint16_t* gr = reinterpret_cast<const uint16_t*>(weights + w_norm);
     struct Frag {
       u32x4_t w[CT], gn;
       f4v xlo[NT], xhi[NT];
@@ -303,9 +392,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     auto load = [&](int k, Frag& f) {
 #pragma unroll
       for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
-      f.gn = u32x4_t{0u, 0u, 0u, 0u};
-      if constexpr (kNorm)
-        if (k + 8 * g < width) f.gn = gload16(gr + k);
+      if constexpr (kNorm) f.gn = gload16(gr + norm_at(k + 8 * g, 8));
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const float* p = xr + ((size_t)t * nkb + k / 32) * 512;
@@ -357,7 +444,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
       }
       if constexpr (kNorm) pin4(f.gn);
     };
-    k_loop<SW, 32, NT * CT <= 2, Frag>(first, slice, load, pin, mma);
+    k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, early);
   } else {
     // Mixed mode: the operand is an FP16 buffer (its values are cast points) and the weights
     // are FP16; one v_mfma_f32_16x16x32_f16 per 32-k block, lane (r16, g) holding
@@ -389,7 +476,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
 #pragma unroll
       for (int t = 0; t < NT; t++) pin4(f.x[t]);
     };
-    k_loop<SW, 32, NT * CT <= 2, Frag>(first, slice, load, pin, mma);
+    k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, early);
   }
   // A wave holding two slices adds them here: the first level of the tree.
 #pragma unroll
@@ -408,28 +495,24 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     }
   }
   __syncthreads();
-  // Epilogue: one thread per output unit (a column, or the column pair of a RoPE pair /
-  // gate-up pair) of a stream below B.
-  constexpr int unit = (E == kEpQkv || E == kEpGateUp) ? 2 : 1;
-  constexpr int per_row = kBatchTile * CT / unit;
   auto tree = [&](auto at) {
     float p[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) p[k] = SW == 2 ? at(k) : at(2 * k) + at(2 * k + 1);
     return (p[0] + p[1]) + (p[2] + p[3]);
   };
-  for (int o = threadIdx.x; o < NT * kBatchTile * per_row; o += blockDim.x) {
-    const int t = o / (kBatchTile * per_row);
-    const int row = (o / per_row) % kBatchTile;
-    const int cc = (o % per_row) * unit;
-    const int c = cc / kBatchTile, col = cc % kBatchTile;
-    const int b = (t0 + t) * kBatchTile + row;
-    if (b >= a.streams) continue;
-    float s0 = tree([&](int k) { return red[k][t][c][row][col]; });
-    float s1 = unit == 2 ? tree([&](int k) { return red[k][t][c][row][col + 1]; }) : 0.f;
+#pragma unroll
+  for (int u = 0; u < kOwn; u++) {
+    if (!owned(u)) break;
+    const Unit o = unit_of(u);
+    const int b = (t0 + o.t) * kBatchTile + o.row;
+    if (b >= streams) continue;
+    const int c = o.cc / kBatchTile, col = o.cc % kBatchTile;
+    float s0 = tree([&](int k) { return red[k][o.t][c][o.row][col]; });
+    float s1 = unit == 2 ? tree([&](int k) { return red[k][o.t][c][o.row][col + 1]; }) : 0.f;
     if constexpr (kNorm) {
-      const float sum = tree([&](int k) { return sq[k][t][row]; });
-      const float scale = 1.0f / sqrtf(sum / (float)a.width + a.epsilon);
+      const float sum = tree([&](int k) { return sq[k][o.t][o.row]; });
+      const float scale = 1.0f / sqrtf(sum / (float)width + epsilon);
       s0 *= scale;
       s1 *= scale;
     }
@@ -437,54 +520,43 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const BatchArgs*
     // does (src/cuda/Primitives.cuh:148-239); cast<P> is the identity for FP32 storage.
     s0 = cast<P>(s0);
     s1 = cast<P>(s1);
-    const int n = n0 + cc;
-    float* xp = a.x + act_index<P>(b, n, a.width_p);  // x[b][n]
+    const int n = n0 + o.cc;
     if constexpr (E == kEpInput) {
-      *xp = s0;
+      reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = s0;
     } else if constexpr (E == kEpQkv) {
       // src/cuda/Primitives.cuh:148-166: RoPE on adjacent pairs of q and k, then the ring write.
-      const int sec = (n >= a.width) + (n >= 2 * a.width);
-      const int i = n - sec * a.width;
-      const unsigned long long pos = a.position[b];
+      const int sec = (n >= width) + (n >= 2 * width);
+      const int i = n - sec * width;
       float va = s0, vb = s1;
       if (sec < 2) {
         // No FMA contraction here: left to the compiler, it fuses one product or the other
         // depending on the kernel variant, and a stream's bits would then depend on the
         // workgroup shape chosen for its batch size.
 #pragma clang fp contract(off)
-        const int e = i % a.dim;
-        const float angle = (float)pos * a.rope_freq[e >> 1];
-        const float co = cosf(angle), si = sinf(angle);
-        const float ra = va * co - vb * si, rb = va * si + vb * co;
+        const float ra = va * cs[u].x - vb * cs[u].y, rb = va * cs[u].y + vb * cs[u].x;
         va = cast<P>(ra);
         vb = cast<P>(rb);
       }
-      if (sec == 0) {
-        a.q[(size_t)b * a.width + i] = va;
-        a.q[(size_t)b * a.width + i + 1] = vb;
+      const int h = i / dim, d = i - h * dim;
+      const size_t dst = sec == 0 ? (size_t)b * width + i
+                                  : ((((size_t)layer * streams + b) * heads + h) * window + slot[u]) * dim + d;
+      float* base = sec == 0 ? qkv_q : sec == 1 ? qkv_k : qkv_v;
+      if (P == kMixed && sec != 0) {
+        *in_global(reinterpret_cast<unsigned*>(reinterpret_cast<uint16_t*>(base) + dst)) =
+            (unsigned)float_to_half(va) | ((unsigned)float_to_half(vb) << 16);
       } else {
-        const int h = i / a.dim, d = i - h * a.dim;
-        const int slot = (int)(pos % (unsigned long long)a.window);
-        const size_t ring = ((((size_t)layer * a.streams + b) * a.heads + h) * a.window + slot) * a.dim + d;
-        void* dst = sec == 1 ? a.keys : a.values;
-        if constexpr (P == kMixed) {
-          reinterpret_cast<uint16_t*>(dst)[ring] = float_to_half(va);
-          reinterpret_cast<uint16_t*>(dst)[ring + 1] = float_to_half(vb);
-        } else {
-          reinterpret_cast<float*>(dst)[ring] = va;
-          reinterpret_cast<float*>(dst)[ring + 1] = vb;
-        }
+        *in_global(reinterpret_cast<v2f*>(base + dst)) = v2f{va, vb};
       }
     } else if constexpr (E == kEpOut) {
-      *xp = cast<P>(*xp + s0);
+      reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = cast<P>(res[u] + s0);
     } else if constexpr (E == kEpGateUp) {
       const float v = cast<P>((s0 / (1.0f + expf(-s0))) * s1);
-      if constexpr (P == kMixed) reinterpret_cast<uint16_t*>(a.act)[half_index(b, n >> 1, a.ffn_p)] = float_to_half(v);
-      else a.act[act_index<P>(b, n >> 1, a.ffn_p)] = v;
+      if constexpr (P == kMixed) reinterpret_cast<uint16_t*>(out)[half_index(b, n >> 1, out_ld)] = float_to_half(v);
+      else reinterpret_cast<float*>(out)[act_index<P>(b, n >> 1, out_ld)] = v;
     } else {
-      const float v = cast<P>(*xp + s0);
-      *xp = v;
-      a.hidden[((size_t)b * a.layers + layer) * a.width + n] = v;
+      const float v = cast<P>(res[u] + s0);
+      reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = v;
+      in_global(hidden)[((size_t)b * layers + layer) * width + n] = v;
     }
   }
 }
