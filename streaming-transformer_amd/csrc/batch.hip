@@ -98,6 +98,11 @@ Batch::Batch(const st_config& config, bool mixed, const st_tensor* tensors, size
   a.act = zeroed(act_, (size_t)streams_p_ * a.ffn_p);
   a.q = zeroed(q_, (size_t)streams_p_ * a.width);
   a.score = zeroed(score_, (size_t)streams_);
+  if (attn_split()) {
+    const int row = 64 * (dim_ > 64 ? 2 : 1) + 2;
+    attn_part_.alloc((size_t)streams_ * c_.heads * attn_chunks() * row * 4);
+    zeroed(attn_count_, (size_t)streams_ * c_.heads);
+  }
   a.rope = reinterpret_cast<float2*>(zeroed(step_rope_, (size_t)streams_p_ * dim_));
   a.slot = reinterpret_cast<int*>(zeroed(step_slot_, (size_t)streams_p_));
   host_in_.alloc((size_t)streams_p_ * a.features_p * 4);
@@ -158,6 +163,51 @@ void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff,
   else ring(std::integral_constant<int, 1>{});
 }
 
+// Attention of one layer. Windows of more than one chunk: a workgroup per (stream, head, chunk)
+// where the (stream, head) pairs alone give fewer than kSplitPairs workgroups, one per CU (or the
+// window has more chunks than one workgroup keeps), else one that walks its chunks. Split, Main
+// with W = 1024 at 4 streams (32 pairs) went 249 -> 199 us per step; above the line a merge costs
+// more than the spread gives: 296 pairs of two chunks 111.8 us walked, 114.2 split; Large at 32
+// streams (512 pairs of four) 574 walked, 586 split.
+template <int P, bool kNT>
+void Batch::attend(int layer) {
+  const size_t block = (size_t)c_.width * c_.window * (P == kMixed ? 2 : 4);  // a (layer, stream) block in bytes
+  const char* keys = reinterpret_cast<const char*>(args_.keys) + (size_t)layer * streams_ * block;
+  const char* values = reinterpret_cast<const char*>(args_.values) + (size_t)layer * streams_ * block;
+  if (dim_ > 128) {
+    hipLaunchKernelGGL((batch_attention_wide<P, kNT>), dim3(c_.heads, streams_), dim3(kAttnThreads), (size_t)c_.window * 4,
+                       stream_, args_.position, args_.q, keys, values, args_.attn, c_.window, dim_, c_.heads, args_.width_p);
+    return;
+  }
+  const int chunks = attn_chunks();
+  const bool split = attn_split();
+  auto go = [&](auto kernel, int dv) {
+    const size_t lds = (size_t)(split ? 1 : chunks) * kAttnWaves * (64 * dv + 2) * 4;
+    hipLaunchKernelGGL(kernel, dim3(c_.heads, streams_, split ? chunks : 1), dim3(kAttnThreads), lds, stream_, args_.position,
+                       args_.q, keys, values, args_.attn, c_.window, dim_, c_.heads, args_.width_p,
+                       reinterpret_cast<float*>(attn_part_.ptr), reinterpret_cast<unsigned*>(attn_count_.ptr));
+  };
+  // The loads that do not wait for the position read every slot of the window: for one-chunk
+  // windows whose rings stay cached and that are too few to fill the chip (elsewhere the unwritten
+  // slots' bytes would cost more than the round trip).
+  const bool any = !kNT && chunks == 1 && streams_ * c_.heads <= kSplitPairs;
+  auto form = [&](auto DV, auto NP) {
+    constexpr int dv = decltype(DV)::value, np = decltype(NP)::value;
+    if constexpr (!kNT) {
+      if (any) return go(batch_attention<P, dv, np, true, kNT>, dv);
+    }
+    go(batch_attention<P, dv, np, false, kNT>, dv);
+  };
+  using std::integral_constant;
+  if (dim_ > 64) {
+    if (c_.window <= 64) form(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    else form(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+  } else {
+    if (c_.window <= 64) form(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    else form(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+  }
+}
+
 // Workgroup shapes per projection. Every shape computes the same fixed slice tree, so the
 // choice changes speed only, never a stream's bits. Small batches want many workgroups (one
 // column tile and one K-slice per wave); large ones want each X fragment reused across column
@@ -174,10 +224,6 @@ void Batch::launch_sequence() {
   const int d = c_.width, F = c_.ffn;
   const bool wide = streams_p_ >= 64, narrow = streams_p_ >= 128 && (c_.width / kBatchTile) % 2 == 0;
   const bool huge = P != kFp32 && streams_p_ >= 256;
-  // The attention loops' form (batch_attention): chunked loads for dh <= 64, eight passes with
-  // V loaded early up to 32 streams, four with V early at 64, four from 128.
-  const int attn_loads = dim_ > 64 ? kAttnPerPass
-                         : streams_p_ <= 32 ? kAttnChunk8Early : streams_p_ == 64 ? kAttnChunk4Early : kAttnChunk4;
   // K/V rings that do not fit in the Infinity Cache beside the weights are read with
   // non-temporal loads, so that the weights stay cached.
   const bool kv_nt = 2 * c_.layers * (size_t)streams_ * block_words_ * 4 + offsets_.weight_bytes > kInfinityCacheBytes;
@@ -196,23 +242,8 @@ void Batch::launch_sequence() {
     if (wide && wide_qkv_)
       project<P, kEpQkv, kFold, 2, 2>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l, huge ? 1 : kGroupTiles);
     else project<P, kEpQkv, kFold, 1, 1>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
-    {
-      const dim3 grid(streams_ * c_.heads), block(kAttnThreads);
-      const size_t lds = (size_t)c_.window * 4;
-      auto attend = [&](auto nt) {
-        constexpr bool kNT = decltype(nt)::value;
-        if (attn_loads == kAttnChunk4)
-          hipLaunchKernelGGL((batch_attention<P, kAttnChunk4, kNT>), grid, block, lds, stream_, dargs_, l);
-        else if (attn_loads == kAttnChunk4Early)
-          hipLaunchKernelGGL((batch_attention<P, kAttnChunk4Early, kNT>), grid, block, lds, stream_, dargs_, l);
-        else if (attn_loads == kAttnChunk8Early)
-          hipLaunchKernelGGL((batch_attention<P, kAttnChunk8Early, kNT>), grid, block, lds, stream_, dargs_, l);
-        else
-          hipLaunchKernelGGL((batch_attention<P, kAttnPerPass, kNT>), grid, block, lds, stream_, dargs_, l);
-      };
-      if (kv_nt) attend(std::true_type{});
-      else attend(std::false_type{});
-    }
+    if (kv_nt) attend<P, true>(l);
+    else attend<P, false>(l);
     if (narrow) project<P, kEpOut, false, 2, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
     else project<P, kEpOut, false, 1, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
     norm(w.norm2);

@@ -43,6 +43,14 @@ class Batch : public BatchBase {
     else HIP_CHECK(hipGraphLaunch(graph_exec_, stream_));
   }
   template <int P> void launch_sequence();
+  template <int P, bool kNT> void attend(int layer);
+  // Chunks of the attention window, and whether they are spread over workgroups (batch_attention).
+  static constexpr int kSplitPairs = 256;
+  int attn_chunks() const { return (c_.window + kBatchChunk - 1) / kBatchChunk; }
+  bool attn_split() const {
+    const int chunks = attn_chunks();
+    return dim_ <= 128 && chunks > 1 && (chunks > kAttnLoop || streams_ * c_.heads < kSplitPairs);
+  }
   template <int P, int E, bool kNorm, int CT, int SW>
   void project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer,
                int max_tiles = kGroupTiles);
@@ -63,7 +71,7 @@ class Batch : public BatchBase {
   GraphHandle graph_;
   GraphExecHandle graph_exec_;
   DeviceBuffer weights_, keys_, values_, hidden_, position_, in_, x_, xn_, attn_, act_, q_, score_, rope_, step_rope_, step_slot_,
-      args_dev_;
+      args_dev_, attn_part_, attn_count_;
   PinnedBuffer host_in_, host_out_;
   StepArgs offsets_{};  // weight arena offsets (shared layout with the single-stream runtime)
   BatchArgs args_{};

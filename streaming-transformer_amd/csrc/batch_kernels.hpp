@@ -179,6 +179,7 @@ __device__ __forceinline__ void k_ring(int first, int slice, Load&& load, Pin&& 
 
 __device__ __forceinline__ void pin4(u32x4_t& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin4(f4v& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void pin4(u32x2_t& v) { asm volatile("" : "+v"(v)); }
 
 // One projection Y = X . W^T over the batch, with its phase's epilogue. Workgroup: CT column
 // tiles of 16 outputs and NT batch tiles of 16 streams. K is cut into 8 slices; each wave
@@ -583,184 +584,305 @@ __device__ __forceinline__ float4 ring4(const void* ring, size_t i) {
 // The chunked attention keeps the loaded form in registers and widens at each use, so that the
 // FP16 values feed mixed-precision FMAs directly (widening is exact, the results unchanged).
 template <int P>
-using RingRaw = std::conditional_t<P == kMixed, uint2, float4>;
+using RingRaw = std::conditional_t<P == kMixed, u32x2_t, f4v>;
 template <int P, bool kNT>
 __device__ __forceinline__ RingRaw<P> ring_raw(const void* ring, size_t i) {
   typedef const __attribute__((address_space(1))) u32x2_t g2;
   typedef const __attribute__((address_space(1))) u32x4_t g4;
   if constexpr (P == kMixed) {
     const void* p = reinterpret_cast<const uint16_t*>(ring) + i;
-    return __builtin_bit_cast(uint2, kNT ? __builtin_nontemporal_load((g2*)p) : *(g2*)p);
+    return kNT ? __builtin_nontemporal_load((g2*)p) : *(g2*)p;
   } else {
-    return ring4<P, kNT>(ring, i);
+    return __builtin_bit_cast(f4v, ring4<P, kNT>(ring, i));
   }
 }
-__device__ __forceinline__ const float4& widen(const float4& v) { return v; }
-__device__ __forceinline__ float4 widen(uint2 h) {
-  return make_float4(half_to_float((unsigned short)(h.x & 0xffffu)), half_to_float((unsigned short)(h.x >> 16)),
-                     half_to_float((unsigned short)(h.y & 0xffffu)), half_to_float((unsigned short)(h.y >> 16)));
+__device__ __forceinline__ f4v widen(f4v v) { return v; }
+__device__ __forceinline__ f4v widen(u32x2_t h) {
+  return f4v{half_to_float((unsigned short)(h.x & 0xffffu)), half_to_float((unsigned short)(h.x >> 16)),
+             half_to_float((unsigned short)(h.y & 0xffffu)), half_to_float((unsigned short)(h.y >> 16))};
 }
 
 constexpr int kAttnThreads = 256;  // batch_attention's workgroup: four waves, 16 groups of 16 lanes
+constexpr int kAttnWaves = kAttnThreads / 64;
+constexpr int kBatchChunk = 128;    // ring slots per attention chunk
+constexpr int kAttnLoop = 8;       // most chunks that one workgroup walks (its partials are in LDS)
 
-// batch_attention for dh <= 64: lane (group grp, r) holds elements 4r .. 4r + 3 of its rows,
-// one 16-byte load per row, the loads of NP passes of 16 rows issued together; with kEarlyV the
-// first chunk's V loads are issued before the softmax reductions. The arithmetic is the general
-// loop's, in the same order: per row a dot product over the lane's four elements and a 16-lane
-// sum; per group the V rows of slots grp, grp + 16, ... accumulated in slot order.
-template <int P, int NP, bool kEarlyV, bool kNT>
-__device__ __forceinline__ void attention_chunked(const BatchArgs& a, int b, int h, int valid, size_t base,
-                                                  const float* q, float div, float* pr, float* wred,
-                                                  float4 (*vred)[17]) {
-  constexpr int kRows = 16 * NP;
-  const int dim = a.dim;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = tid & 15, grp = tid >> 4;
-  const int d = 4 * r;
-  const bool in = d < dim;
-  const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  const float4 qv = in ? *reinterpret_cast<const float4*>(q + d) : z4;
-  // Slots past `valid` load slot valid - 1 and are dropped.
-  auto at = [&](int s) { return base + (size_t)(s < valid ? s : valid - 1) * dim + d; };
-  // V rows of a chunk; filled in place (an array filled through a lambda went to scratch).
-  // K and V stay in their loaded form (RingRaw) until used.
-  const RingRaw<P> zr{};
-  RingRaw<P> vv[NP];
-  float mx = -INFINITY;
-  for (int c0 = 0; c0 < valid; c0 += kRows) {
-    RingRaw<P> kv[NP];
-#pragma unroll
-    for (int p = 0; p < NP; p++) kv[p] = in ? ring_raw<P, kNT>(a.keys, at(c0 + 16 * p + grp)) : zr;
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-      const int s = c0 + 16 * p + grp;
-      float dot = 0.f;
-      if (in) {
-        const float4& k = widen(kv[p]);
-        dot += qv.x * k.x;
-        dot += qv.y * k.y;
-        dot += qv.z * k.z;
-        dot += qv.w * k.w;
-      }
-      dot = group_sum(dot, 16);
-      if (s < valid) {
-        const float lg = dot / div;
-        if (r == 0) pr[s] = lg;
-        mx = fmaxf(mx, lg);
-      }
-    }
-  }
-  if constexpr (kEarlyV) {
-#pragma unroll
-    for (int p = 0; p < NP; p++) vv[p] = in ? ring_raw<P, kNT>(a.values, at(16 * p + grp)) : zr;
-  }
-  mx = wave_top(mx);
-  if (lane == 0) wred[wave] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(wred[0], wred[1]), fmaxf(wred[2], wred[3]));
-  float sum = 0.f;
-  for (int s = tid; s < valid; s += kAttnThreads) {
-    const float e = expf(pr[s] - mx);
-    pr[s] = e;
-    sum += e;
-  }
-  sum = wave_total(sum);
-  __syncthreads();  // every wave has read wred (max) and written its probabilities
-  if (lane == 0) wred[wave] = sum;
-  __syncthreads();
-  sum = (wred[0] + wred[1]) + (wred[2] + wred[3]);
-  float4 o = z4;
-  for (int c0 = 0; c0 < valid; c0 += kRows) {
-    if (!kEarlyV || c0 > 0) {
-#pragma unroll
-      for (int p = 0; p < NP; p++) vv[p] = in ? ring_raw<P, kNT>(a.values, at(c0 + 16 * p + grp)) : zr;
-    }
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-      const int s = c0 + 16 * p + grp;
-      if (s < valid) {
-        const float pp = pr[s];
-        const float4& v = widen(vv[p]);
-        o.x += pp * v.x;
-        o.y += pp * v.y;
-        o.z += pp * v.z;
-        o.w += pp * v.w;
-      }
-    }
-  }
-  vred[grp][r] = o;
-  __syncthreads();
-  if (tid < 16 && 4 * tid < dim) {
-    float4 acc = vred[0][tid];
-    for (int k = 1; k < 16; k++) {
-      const float4 v = vred[k][tid];
-      acc.x += v.x;
-      acc.y += v.y;
-      acc.z += v.z;
-      acc.w += v.w;
-    }
-    const float o4[4] = {acc.x / sum, acc.y / sum, acc.z / sum, acc.w / sum};
-    // attn[b][h dh + 4 tid + j]: four consecutive elements in the tiled layouts too.
-    const int n = h * dim + 4 * tid;
-    const size_t oi = P == kMixed ? half_index(b, n, a.width_p) : act_index<P>(b, n, a.width_p);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      if constexpr (P == kMixed) reinterpret_cast<uint16_t*>(a.attn)[oi + j] = float_to_half(o4[j]);
-      else a.attn[oi + j] = o4[j];
-    }
-  }
+// Weight of a softmax partial with maximum m beside the overall maximum `top`. A partial without
+// finite logits (m = -inf) carries zeros and gets weight zero; if every logit is -inf the sum is
+// zero and the output 0 / 0, as a softmax over them has it.
+__device__ __forceinline__ float partial_weight(float m, float top) { return m == -INFINITY ? 0.f : expf(m - top); }
+
+// One element of the attention output, [b][n] of the padded rows.
+template <int P>
+__device__ __forceinline__ void put_attn(void* attn, int b, int n, int width_p, float v) {
+  if constexpr (P == kMixed) in_global(reinterpret_cast<uint16_t*>(attn))[half_index(b, n, width_p)] = float_to_half(v);
+  else in_global(reinterpret_cast<float*>(attn))[act_index<P>(b, n, width_p)] = v;
 }
 
 // Attention of one (stream, head) over the stream's valid ring slots [0, valid)
 // (src/cuda/Primitives.cuh:167-219): logits q.K/sqrt(dh), softmax, weighted V, cast. Slot order
-// does not change the result beyond summation order. Four waves; every load is a coalesced
-// row:
-//  - logits: 16 lanes per K row (4 elements each, rows of up to 64 elements per pass), a
-//    16-lane DPP sum, so a wave covers 4 rows per load;
-//  - softmax: workgroup max and sum through LDS;
-//  - values: lane group (slot s mod 16) accumulates its slots' V rows, 4 elements per lane,
-//    and the 16 groups are summed in LDS in group order.
-// Needs dh a multiple of 4; dynamic LDS holds `window` floats of probabilities. The rings are
-// layer-major, so a layer's K and V are one contiguous region. kLoads picks the form of the
-// loops, on the host, by storage and batch size; every form computes the same values in the same
-// order, so a stream's bits do not depend on it:
-//  - kAttnPerPass: the general loop below, one pass of 16 rows after the other (any dh);
-//  - kAttnChunk4, kAttnChunk4Early, kAttnChunk8Early: dh <= 64, the loads of 4 or 8 passes
-//    issued together (attention_chunked); the Early forms load the first V chunk before the
-//    softmax.
-// Measured on Main (one layer, W = 128): with FP32 K/V at 256 streams 23.2 us against 26.2 us
-// for the per-pass loop in the former stream-major layout, at 64 streams 6.95 (4, early V)
-// against 8.8, at 16 streams 5.2 (8) against 7.4 (and 8 with early V, once the K/V loads were
-// global loads, 183.7 -> 181.2 us per Main step). FP16 K/V take the same forms since the
-// chunked loops keep K and V in their loaded form (RingRaw) until each use: converted when
-// loaded, they were slower than the per-pass loop below 256 streams (at 16 streams 9.7-10.4
-// against 7.9 us per layer); kept as loaded, Main mixed steps went 204 -> 187 us at one stream,
-// 214 -> 200 at 16, 237 -> 226 at 64 and 368 -> 344 at 256.
+// does not change the result beyond summation order. Head dims up to 64 DV (DV 1 or 2), a
+// multiple of 4.
+//
+// The window is cut into chunks of kBatchChunk slots. 16 lanes share a K (or V) row, 4 DV elements
+// each, so a wave's load covers 4 rows; a wave owns 4 rows of each of the NP passes of 16 rows,
+// and the chunk's K and V loads are all issued before the first dot product (NP = 8; windows of
+// at most 64 slots take NP = 4). Each wave forms its own softmax partial of a chunk: its rows'
+// maximum m, s = sum exp(l - m), o = sum exp(l - m) V, in registers. One barrier, then wave 0 merges
+// the four waves' partials of each chunk, and the chunks in order. So the critical path of a
+// one-chunk window is: position, K and V in one round trip, one barrier. (Before: the arguments
+// block, then the position, then K; a maximum, a sum and an output through LDS with five
+// barriers. Main with bfloat16 weights at 16 streams 188.7 -> 178.4 us per step, at 256 430.6 ->
+// 425.5; mixed mode at 64 streams 243.2 -> 239.3.)
+//
+// Workgroups: gridDim.z == 1: one walks all chunks of its (stream, head), its partials in LDS.
+// Otherwise workgroup z takes chunk z, writes the chunk's partial through to memory and counts
+// itself; the last to arrive merges the chunks (it finds every partial there: nothing waits).
+// Both run the same arithmetic in the same order, so a stream's bits do not depend on the form,
+// which the host picks by how many workgroups the (stream, head) pairs alone would give.
+//
+// kAny: the first loads clamp rows to the window instead of to the valid slots, so that they do
+// not wait for the position (slots not yet written hold the zeros of the reset and are dropped).
 // kNT: the K and V loads are non-temporal, for rings that do not fit in the Infinity Cache
 // beside the weights: a step streams them through once, and cached they would evict the
 // weights the projections re-read (Main, bfloat16 weights: 454 -> 436 us per step at 256
 // streams, 249 -> 241 at 64; mixed mode 400 -> 382 at 256). Rings that fit stay cached from
 // step to step instead (mixed mode at 64 streams: 253 against 270 us).
-enum AttnLoads : int { kAttnPerPass = 0, kAttnChunk4, kAttnChunk4Early, kAttnChunk8Early };
-template <int P, int kLoads, bool kNT>
-__global__ __launch_bounds__(kAttnThreads) void batch_attention(const BatchArgs* __restrict__ ap, int layer) {
-  const BatchArgs& a = *ap;
+template <int P, int DV, int NP, bool kAny, bool kNT>
+__global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned long long* __restrict__ position,
+                                                                const float* __restrict__ q, const void* keys,
+                                                                const void* values, void* attn, int window, int dim,
+                                                                int heads, int width_p, float* partial,
+                                                                unsigned* arrived) {
+  extern __shared__ float part[];  // [chunk][wave][64 DV + 2]: o, then m and s
+  constexpr int kRow = 64 * DV + 2;
+  const int h = blockIdx.x, b = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = tid & 15, grp = tid >> 4;
+  const int d = 4 * r;
+  const size_t base = ((size_t)b * heads + h) * (size_t)window * dim;
+  const bool split = gridDim.z > 1;
+  const int first = split ? (int)blockIdx.z : 0;
+  const float div = sqrtf((float)dim);
+  // K and V stay in their loaded form (RingRaw: FP16 pairs in mixed mode) until used. Lanes past
+  // the head dim load the row's last elements and drop them.
+  RingRaw<P> kv[NP][DV], vv[NP][DV];
+  int dd[DV];
+  f4v qv[DV];
+#pragma unroll
+  for (int j = 0; j < DV; j++) {
+    dd[j] = d + 64 * j < dim ? d + 64 * j : dim - 4;
+    qv[j] = gload16f(q + ((size_t)b * heads + h) * dim + dd[j]);
+  }
+  auto load = [&](const void* ring, RingRaw<P> (&f)[NP][DV], int c0, int limit) {
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const int s = c0 + 16 * p + grp;
+      const size_t row = base + (size_t)(s < limit ? s : limit - 1) * dim;
+#pragma unroll
+      for (int j = 0; j < DV; j++) f[p][j] = ring_raw<P, kNT>(ring, row + dd[j]);
+    }
+    asm volatile("" ::: "memory");  // the loads stay here, ahead of the arithmetic
+  };
+  int valid = window;
+  if constexpr (!kAny) {
+    const unsigned long long t = position[b];
+    valid = t + 1 < (unsigned long long)window ? (int)(t + 1) : window;
+    if (first * kBatchChunk >= valid) return;
+  }
+  load(keys, kv, first * kBatchChunk, valid);
+  load(values, vv, first * kBatchChunk, valid);
+  if constexpr (kAny) {
+    const unsigned long long t = position[b];
+    valid = t + 1 < (unsigned long long)window ? (int)(t + 1) : window;
+  }
+  const int active = (valid + kBatchChunk - 1) / kBatchChunk;  // chunks with valid slots
+  const int last = split ? first + 1 : active;
+  // One chunk; with `more` its registers are reloaded with the next chunk's rows as soon as they are
+  // used, without a condition (a conditional load came out as a register copy per element at the
+  // end of the round, which waited for every load). The pins keep each row's arithmetic after
+  // its own load.
+  auto chunk = [&](int c, auto more) {
+    const int c0 = c * kBatchChunk;
+    float lg[NP], mx = -INFINITY;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      float dot = 0.f;
+#pragma unroll
+      for (int j = 0; j < DV; j++) {
+        pin4(kv[p][j]);
+        const f4v k = widen(kv[p][j]);
+        float part_dot = __builtin_fmaf(qv[j].x, k.x, dot);
+        part_dot = __builtin_fmaf(qv[j].y, k.y, part_dot);
+        part_dot = __builtin_fmaf(qv[j].z, k.z, part_dot);
+        part_dot = __builtin_fmaf(qv[j].w, k.w, part_dot);
+        dot = d + 64 * j < dim ? part_dot : dot;
+      }
+      dot = group_sum(dot, 16);
+      float l = dot / div;
+      asm volatile("" : "+v"(l));  // no branch around the division
+      lg[p] = c0 + 16 * p + grp < valid ? l : -INFINITY;
+      mx = fmaxf(mx, lg[p]);
+    }
+    if constexpr (more.value) load(keys, kv, c0 + kBatchChunk, valid);
+    mx = wave_top(mx);
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    float sum = 0.f;
+    f4v o[DV];
+#pragma unroll
+    for (int j = 0; j < DV; j++) o[j] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const float e = expf(lg[p] - ref);
+      sum += e;
+      const bool live = c0 + 16 * p + grp < valid;
+#pragma unroll
+      for (int j = 0; j < DV; j++) {
+        pin4(vv[p][j]);
+        const f4v v = widen(vv[p][j]);
+        o[j].x = live ? __builtin_fmaf(e, v.x, o[j].x) : o[j].x;
+        o[j].y = live ? __builtin_fmaf(e, v.y, o[j].y) : o[j].y;
+        o[j].z = live ? __builtin_fmaf(e, v.z, o[j].z) : o[j].z;
+        o[j].w = live ? __builtin_fmaf(e, v.w, o[j].w) : o[j].w;
+      }
+    }
+    if constexpr (more.value) load(values, vv, c0 + kBatchChunk, valid);
+    sum = column_sum(sum, 16);
+    float* mine = part + ((c - first) * kAttnWaves + wave) * kRow;
+#pragma unroll
+    for (int j = 0; j < DV; j++) {
+      o[j].x = column_sum(o[j].x, 16);
+      o[j].y = column_sum(o[j].y, 16);
+      o[j].z = column_sum(o[j].z, 16);
+      o[j].w = column_sum(o[j].w, 16);
+      if (lane < 16) {
+        mine[64 * j + d] = o[j].x;
+        mine[64 * j + d + 1] = o[j].y;
+        mine[64 * j + d + 2] = o[j].z;
+        mine[64 * j + d + 3] = o[j].w;
+      }
+    }
+    if (lane == 0) {
+      mine[64 * DV] = mx;
+      mine[64 * DV + 1] = sum;
+    }
+  };
+  int c = first;
+  for (; c + 1 < last; c++) chunk(c, std::true_type{});
+  chunk(c, std::false_type{});
+  __syncthreads();
+  if (wave != 0) return;
+  // The merges, each lane for its own columns lane + 64 j. No FMA contraction: both forms must
+  // round alike.
+  auto merge_waves = [&](int c, float& m, float& s, float (&o)[DV]) {
+    const float* w = part + c * kAttnWaves * kRow;
+    float mw[4], e[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) mw[k] = w[k * kRow + 64 * DV];
+    m = fmaxf(fmaxf(mw[0], mw[1]), fmaxf(mw[2], mw[3]));
+#pragma unroll
+    for (int k = 0; k < 4; k++) e[k] = partial_weight(mw[k], m);
+    auto sum4 = [&](int i) {
+#pragma clang fp contract(off)
+      return (w[i] * e[0] + w[kRow + i] * e[1]) + (w[2 * kRow + i] * e[2] + w[3 * kRow + i] * e[3]);
+    };
+    s = sum4(64 * DV + 1);
+#pragma unroll
+    for (int j = 0; j < DV; j++) o[j] = sum4(lane + 64 * j);
+  };
+  auto put = [&](const float (&num)[DV], float den) {
+#pragma unroll
+    for (int j = 0; j < DV; j++)
+      if (lane + 64 * j < dim) put_attn<P>(attn, b, h * dim + lane + 64 * j, width_p, num[j] / den);
+  };
+  float m, s, o[DV];
+  if (active == 1) {
+    merge_waves(0, m, s, o);
+    put(o, s);
+    return;
+  }
+  float num[DV], den = 0.f, top = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < DV; j++) num[j] = 0.f;
+  auto add_chunk = [&](float mc, float sc, const float (&oc)[DV]) {
+#pragma clang fp contract(off)
+    const float e = partial_weight(mc, top);
+    den = den + sc * e;
+#pragma unroll
+    for (int j = 0; j < DV; j++) num[j] = num[j] + oc[j] * e;
+  };
+  if (!split) {
+    for (int k = 0; k < active * kAttnWaves; k++) top = fmaxf(top, part[k * kRow + 64 * DV]);
+    for (int c = 0; c < active; c++) {
+      merge_waves(c, m, s, o);
+      add_chunk(m, s, o);
+    }
+    put(num, den);
+    return;
+  }
+  // This chunk's partial, written through to memory (agent scope) and complete before the count.
+  merge_waves(0, m, s, o);
+  const int chunks = (int)gridDim.z, pair = b * heads + h;
+  float* mine = partial + ((size_t)pair * chunks) * kRow;
+  auto at = [&](int c, int i) { return in_global(mine + (size_t)c * kRow + i); };
+#pragma unroll
+  for (int j = 0; j < DV; j++)
+    __hip_atomic_store(at(first, lane + 64 * j), o[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (lane == 0) {
+    __hip_atomic_store(at(first, 64 * DV), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(at(first, 64 * DV + 1), s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  unsigned before = 0;
+  if (lane == 0) before = __hip_atomic_fetch_add(arrived + pair, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  before = __builtin_amdgcn_readfirstlane(before);
+  if (before + 1 != (unsigned)active) return;
+  asm volatile("" ::: "memory");
+  if (lane == 0) __hip_atomic_store(arrived + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  auto get = [&](int c, int i) { return __hip_atomic_load(at(c, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  // Up to kAttnLoop chunks in one round trip, any others (windows over 1024 slots) after it.
+  constexpr int kAhead = kAttnLoop;
+  float mc[kAhead], sc[kAhead], oc[kAhead][DV];
+#pragma unroll
+  for (int c = 0; c < kAhead; c++) {
+    const int cc = c < active ? c : active - 1;
+    mc[c] = get(cc, 64 * DV);
+    sc[c] = get(cc, 64 * DV + 1);
+#pragma unroll
+    for (int j = 0; j < DV; j++) oc[c][j] = get(cc, lane + 64 * j);
+  }
+#pragma unroll
+  for (int c = 0; c < kAhead; c++) top = fmaxf(top, mc[c]);
+  for (int c = kAhead; c < active; c++) top = fmaxf(top, get(c, 64 * DV));
+#pragma unroll
+  for (int c = 0; c < kAhead; c++)
+    if (c < active) add_chunk(mc[c], sc[c], oc[c]);
+  for (int c = kAhead; c < active; c++) {
+#pragma unroll
+    for (int j = 0; j < DV; j++) o[j] = get(c, lane + 64 * j);
+    add_chunk(get(c, 64 * DV), get(c, 64 * DV + 1), o);
+  }
+  put(num, den);
+}
+
+// The same attention for head dims above 128: four waves walk the rows pass by pass, 16 lanes
+// per row in pieces of 64 elements, the softmax maximum and sum through LDS, and the 16 lane groups'
+// V sums added in group order. Dynamic LDS holds `window` floats of probabilities.
+template <int P, bool kNT>
+__global__ __launch_bounds__(kAttnThreads) void batch_attention_wide(const unsigned long long* __restrict__ position,
+                                                                     const float* __restrict__ qs, const void* keys,
+                                                                     const void* values, void* attn, int window, int dim,
+                                                                     int heads, int width_p) {
   extern __shared__ float pr[];
   __shared__ float wred[kAttnThreads / 64];
   __shared__ float4 vred[16][17];
-  const int b = blockIdx.x / a.heads, h = blockIdx.x - b * a.heads;
+  const int h = blockIdx.x, b = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int dim = a.dim, r = tid & 15, grp = tid >> 4;  // 16 groups of 16 lanes
-  const unsigned long long t = a.position[b];
-  const int valid = t + 1 < (unsigned long long)a.window ? (int)(t + 1) : a.window;
-  const size_t base = (((size_t)layer * a.streams + b) * a.heads + h) * (size_t)a.window * dim;
-  const float* q = a.q + (size_t)b * a.width + h * dim;
+  const int r = tid & 15, grp = tid >> 4;  // 16 groups of 16 lanes
+  const unsigned long long t = position[b];
+  const int valid = t + 1 < (unsigned long long)window ? (int)(t + 1) : window;
+  const size_t base = ((size_t)b * heads + h) * (size_t)window * dim;
+  const float* q = qs + ((size_t)b * heads + h) * dim;
   const float div = sqrtf((float)dim);
-  if constexpr (kLoads != kAttnPerPass) {
-    constexpr int np = kLoads == kAttnChunk8Early ? 8 : 4;
-    attention_chunked<P, np, kLoads == kAttnChunk4Early || kLoads == kAttnChunk8Early, kNT>(a, b, h, valid, base, q,
-                                                                                            div, pr, wred, vred);
-    return;
-  }
   float mx = -INFINITY;
   // Rows past `valid` load row valid - 1 and are dropped, so the loop body has no branch
   // around its loads and several passes of loads stay in flight.
@@ -770,7 +892,7 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const BatchArgs*
     const size_t row = base + (size_t)(s < valid ? s : valid - 1) * dim;
     float dot = 0.f;
     for (int d = 4 * r; d < dim; d += 64) {
-      const float4 kv = ring4<P, kNT>(a.keys, row + d);
+      const float4 kv = ring4<P, kNT>(keys, row + d);
       const float4 qv = *reinterpret_cast<const float4*>(q + d);
       dot += qv.x * kv.x;
       dot += qv.y * kv.y;
@@ -806,7 +928,7 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const BatchArgs*
 #pragma unroll 4
       for (int s = grp; s < valid; s += 16) {
         const float p = pr[s];
-        const float4 vv = ring4<P, kNT>(a.values, base + (size_t)s * dim + d);
+        const float4 vv = ring4<P, kNT>(values, base + (size_t)s * dim + d);
         o.x += p * vv.x;
         o.y += p * vv.y;
         o.z += p * vv.z;
@@ -826,12 +948,8 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const BatchArgs*
       }
       const float o4[4] = {acc.x / sum, acc.y / sum, acc.z / sum, acc.w / sum};
       const int n = h * dim + d0 + 4 * tid;
-      const size_t oi = P == kMixed ? half_index(b, n, a.width_p) : act_index<P>(b, n, a.width_p);
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if constexpr (P == kMixed) reinterpret_cast<uint16_t*>(a.attn)[oi + j] = float_to_half(o4[j]);
-        else a.attn[oi + j] = o4[j];
-      }
+      for (int j = 0; j < 4; j++) put_attn<P>(attn, b, n + j, width_p, o4[j]);
     }
     __syncthreads();
   }

@@ -28,7 +28,7 @@ SHAPES = {
     'ref-main': ModelConfig(2, 128, 4, 256, 256, 32),
     # head dim 48
     'dh48': ModelConfig(2, 96, 2, 192, 40, 96),
-    # head dim 128: attention's general per-pass loop (two 64-element passes per row)
+    # head dim 128: attention rows of two 64-element pieces
     'dh128': ModelConfig(2, 256, 2, 512, 48, 256),
     # Large's width and FFN (d = 1024, F = 4096): the longest K-slices and the widest operands
     'wide': ModelConfig(2, 1024, 16, 4096, 40, 1024),
@@ -124,7 +124,43 @@ def test_stream_independent_of_batch(weight_dtype, mixed, streams, steps):
             np.testing.assert_array_equal(x, y)
 
 
-# head dim 128: mixed mode's attention through the per-pass loop
+@pytest.mark.parametrize('dim,heads,window,streams,steps,mixed', [
+    (16, 4, 64, 70, 70, False),     # one chunk of 64 slots
+    (16, 4, 65, 3, 70, False),      # one chunk of 128, loads that do not wait for the position
+    (48, 4, 128, 70, 133, True),    # a full chunk, lanes past the head dim
+    (64, 4, 129, 66, 135, False),   # two chunks, the second of one slot
+    (48, 4, 300, 65, 310, True),    # three chunks
+    (128, 2, 200, 130, 210, False),  # two pieces of 64 elements per row
+    (68, 4, 130, 64, 133, True),    # the second piece of four elements
+    (160, 2, 140, 3, 145, False),   # the wide form
+    (32, 2, 1040, 130, 1050, False),  # nine chunks: split over workgroups for any batch
+])
+def test_attention_chunks_match_a_batch_of_one_and_the_oracle(dim, heads, window, streams, steps, mixed):
+    # A batch of one spreads a window's chunks over workgroups; at 256 or more (stream, head)
+    # pairs one workgroup walks them. Both must give the same bits, before and after the ring wraps.
+    c = ModelConfig(1, dim * heads, heads, 64, window, 24)
+    w = synthetic_checkpoint(c, seed=18, mixed=mixed)
+    events = _events(c, 18, steps, streams)
+    picks = (0, streams - 1)
+    with batch((c, w, mixed), streams) as rt:
+        many = np.stack([rt.step(events[i]) for i in range(steps)])
+        states = [rt.snapshot(b) for b in picks]
+    for b, state in zip(picks, states):
+        oracle = Oracle(c, w, mixed=True) if mixed else Oracle(c, w, accumulate='double')
+        ref = np.array([oracle.step(events[i, b]) for i in range(steps)], dtype=np.float32)
+        if mixed:
+            res = numerical.score_errors(many[:, b], ref, c.layers)
+            assert res['passed'], (b, res)
+        else:
+            assert numerical.fp32_strict_failures(many[:, b], ref, **STRICT) == 0, float(np.abs(many[:, b] - ref).max())
+        with batch((c, w, mixed), 1) as one:
+            alone = np.array([one.step(events[i, b:b + 1])[0] for i in range(steps)], dtype=np.float32)
+            np.testing.assert_array_equal(alone, many[:, b])
+            for x, y in zip(one.snapshot(0), state):
+                np.testing.assert_array_equal(x, y)
+
+
+# head dim 128: attention rows of two 64-element pieces
 @pytest.mark.parametrize('name,streams,steps', [('main', 16, 40), ('small', 19, 90), ('dh128', 6, 60),
                                                 ('wide', 3, 48), ('odd', 5, 60)])
 def test_mixed_streams_meet_the_reference_policy(name, streams, steps):
