@@ -92,7 +92,7 @@ Batch::Batch(const st_config& config, bool mixed, const st_tensor* tensors, size
   HIP_CHECK(hipMemset(position_.ptr, 0, (size_t)streams_ * 8));
   a.position = reinterpret_cast<unsigned long long*>(position_.ptr);
   a.in = zeroed(in_, (size_t)streams_p_ * a.features_p);
-  a.x = zeroed(x_, (size_t)streams_p_ * a.width_p);
+  a.x = zeroed(x_, kSquares + (size_t)streams_p_ * a.width_p) + kSquares;
   a.xn = zeroed(xn_, (size_t)streams_p_ * a.width_p);
   a.attn = zeroed(attn_, (size_t)streams_p_ * a.width_p);
   a.act = zeroed(act_, (size_t)streams_p_ * a.ffn_p);
@@ -227,29 +227,49 @@ void Batch::launch_sequence() {
   // K/V rings that do not fit in the Infinity Cache beside the weights are read with
   // non-temporal loads, so that the weights stay cached.
   const bool kv_nt = 2 * c_.layers * (size_t)streams_ * block_words_ * 4 + offsets_.weight_bytes > kInfinityCacheBytes;
-  // Mixed mode casts each norm's output, so its norms run first into xn; the other modes fold
-  // the norm into the projection (kNorm).
-  constexpr bool kFold = P != kMixed;
-  const void* nx = kFold ? a.x : a.xn;
+  // The norms are folded into the projections (kNorm). Mixed mode casts a norm's output, so a
+  // folding projection converts its X rows (streams x K) again for each of its column tiles (N,
+  // like K the width times a constant); past kFoldWork of them the norms run first, into xn.
+  // Main steps without the fold and with it: 167.7 -> 142.9 us at one stream, 177 -> 144 at 16,
+  // 200 -> 177 at 64, 251 -> 246 at 128, 321 -> 315 at 256; four layers of Large: 134.5 -> 115.5 at
+  // 8, 171.1 -> 171.5 at 32, 221 -> 223 at 64, 325 -> 363 at 128.
+  constexpr size_t kFoldWork = (size_t)256 * 512 * 512;
+  const bool fold = P != kMixed || (size_t)streams_p_ * c_.width * c_.width <= kFoldWork;
+  const void* nx = fold ? a.x : a.xn;
   auto norm = [&](uint32_t w_norm) {
-    if constexpr (!kFold)
-      hipLaunchKernelGGL(batch_norm_mixed, dim3(streams_p_), dim3(256), 0, stream_, dargs_, w_norm);
+    if (!fold) hipLaunchKernelGGL(batch_norm_mixed, dim3(streams_p_), dim3(256), 0, stream_, dargs_, w_norm);
+  };
+  auto qkv_gateup = [&](const LayerWeights& w, int l, auto kFold, auto qkv) {
+    constexpr bool kf = decltype(kFold)::value;
+    if constexpr (decltype(qkv)::value) {
+      if (wide && wide_qkv_)
+        project<P, kEpQkv, kf, 2, 2>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l, huge ? 1 : kGroupTiles);
+      else project<P, kEpQkv, kf, 1, 1>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
+    } else {
+      if (huge && (2 * F / kBatchTile) % 4 == 0)
+        project<P, kEpGateUp, kf, 4, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+      else if (wide && wide_gateup_)
+        project<P, kEpGateUp, kf, 2, 2>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+      else project<P, kEpGateUp, kf, 1, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+    }
+  };
+  auto normed = [&](const LayerWeights& w, int l, auto qkv) {
+    if constexpr (P == kMixed) {
+      if (!fold) return qkv_gateup(w, l, std::false_type{}, qkv);
+    }
+    qkv_gateup(w, l, std::true_type{}, qkv);
   };
   project<P, kEpInput, false, 1, 1>(a.in, a.features_p, a.x, a.width_p, a.w_input, d, 0u, 0);
   for (int l = 0; l < c_.layers; l++) {
     const LayerWeights& w = a.layer[l];
     norm(w.norm1);
-    if (wide && wide_qkv_)
-      project<P, kEpQkv, kFold, 2, 2>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l, huge ? 1 : kGroupTiles);
-    else project<P, kEpQkv, kFold, 1, 1>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
+    normed(w, l, std::true_type{});
     if (kv_nt) attend<P, true>(l);
     else attend<P, false>(l);
     if (narrow) project<P, kEpOut, false, 2, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
     else project<P, kEpOut, false, 1, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
     norm(w.norm2);
-    if (huge && (2 * F / kBatchTile) % 4 == 0) project<P, kEpGateUp, kFold, 4, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
-    else if (wide && wide_gateup_) project<P, kEpGateUp, kFold, 2, 2>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
-    else project<P, kEpGateUp, kFold, 1, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+    normed(w, l, std::false_type{});
     if (narrow) project<P, kEpDown, false, 2, 1>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
     else project<P, kEpDown, false, 1, 1>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
   }

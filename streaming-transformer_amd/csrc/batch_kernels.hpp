@@ -7,8 +7,8 @@
 //    projection prologue;
 //  - mixed (the reference's FP16 mode): FP16 weights and K/V ring, every value rounded to FP16
 //    at the reference's cast points, so each GEMM input is exactly FP16 and runs on
-//    v_mfma_f32_16x16x32_f16 with FP32 accumulation; the norms are materialized (their output
-//    is cast before the projection).
+//    v_mfma_f32_16x16x32_f16 with FP32 accumulation; the norms, whose output is cast before the
+//    projection, are folded into it too, or kernels of their own for large batches.
 // Each stream follows the single-stream runtime's arithmetic up to summation order.
 #pragma once
 
@@ -41,7 +41,7 @@ struct BatchArgs {
   unsigned long long* position;    // [B]
   // Activations, Bp rows of the padded lengths, in the tiled layouts (act_index, half_index):
   float* in;                       // events (features_p)
-  float* x;                        // residual stream (width_p)
+  float* x;                        // residual stream (width_p); mixed mode: kSquares floats before it
   float* xn;                       // normalized x (mixed mode, FP16; width_p)
   float* attn;                     // attention output (FP16 in mixed mode; width_p)
   float* act;                      // SwiGLU output (FP16 in mixed mode; ffn_p)
@@ -52,6 +52,19 @@ struct BatchArgs {
 };
 
 constexpr int kSlices = 8;       // K-slices of a projection, K / 8 columns each
+
+// Mixed mode: the squares of x summed over four columns, kept right before x (so that a kernel
+// with x's address needs no other argument): column quad n / 4 of row b at squares_index.
+constexpr int kSquares = kBatchMax * kMaxDim / 4;
+__host__ __device__ __forceinline__ int squares_index(int b, int quad) {
+  return ((b >> 4) * (kMaxDim / 4) + quad) * 16 + (b & 15);
+}
+// Sum of v * v over each aligned quad of lanes. No contraction: every kernel must round alike.
+__device__ __forceinline__ float quad_squares(float v) {
+#pragma clang fp contract(off)
+  const float s = v * v;
+  return dpp_add<0x4E>(dpp_add<0xB1>(s));
+}
 constexpr size_t kInfinityCacheBytes = (size_t)256 << 20;  // MI355X's memory-side cache (MALL)
 
 // Loads from the weight arena through the global address space. The arena's base arrives in
@@ -202,7 +215,11 @@ __device__ __forceinline__ void pin4(u32x2_t& v) { asm volatile("" : "+v"(v)); }
 // kNorm: X is the residual stream x and the projection consumes RMSNorm(x) . g
 // (src/cuda/Primitives.cuh:122-135). The waves feed x * g to the MFMAs, accumulate the row's
 // sum of squares from the same loads, and the epilogue scales the row by
-// 1 / sqrt(sum / d + eps).
+// 1 / sqrt(sum / d + eps). Mixed mode casts the norm's output, so the scale has to be known before
+// the MFMAs: the kernels that write x also write its squares summed over four columns
+// (kSquares), and each wave adds those of its slice while its first K blocks are in flight. This
+// saves the two norm kernels of a layer (about 2.5 us each) where the conversions that every
+// column tile's workgroup then repeats cost less (Batch::launch_sequence).
 //
 // Everything a kernel needs before its first load comes in the kernel arguments (the first 16
 // dwords are preloaded into SGPRs). What only the epilogue needs (the residual, the RoPE table,
@@ -216,6 +233,8 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
                                                                uint32_t w_norm, int width, int streams, int out_ld,
                                                                int layer) {
   constexpr int kWaves = kSlices / SW, kBlock = 64 * kWaves;
+  constexpr bool kCastNorm = kNorm && P == kMixed;  // the norm's output is cast before the MFMAs
+  constexpr bool kScale = kNorm && P != kMixed;     // the epilogue applies the norm's scale
   const BatchArgs& a = *ap;
   __shared__ float red[kWaves][NT][CT][16][17];
   __shared__ float sq[kWaves][NT][16];
@@ -288,7 +307,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         slot[u] = in_global(slots)[b];
       }
     } else if constexpr (E == kEpGateUp) {
-      if constexpr (kNorm) {
+      if constexpr (kScale) {
         epsilon = a.epsilon;
         asm volatile("" ::"s"(epsilon));
       }
@@ -315,7 +334,13 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
 #pragma unroll
       for (int c = 0; c < CT; c++) acc[i][t][c] = f4v{0.f, 0.f, 0.f, 0.f};
     }
-  static_assert(!(kNorm && P == kMixed), "mixed mode materializes its norms");
+  // The slices' fixed tree over the waves' partials (their pairs already added where SW is 2).
+  auto tree = [&](auto at) {
+    float p[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) p[k] = SW == 2 ? at(k) : at(2 * k) + at(2 * k + 1);
+    return (p[0] + p[1]) + (p[2] + p[3]);
+  };
   // Index of the norm weights of columns k .. k + n - 1. The vector holds `width` values (a
   // multiple of 16); padding columns, whose x is zero, take its last ones, so that the load has
   // no branch around it (one in the K loop's rounds drained every load in flight).
@@ -454,30 +479,107 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
     const int nkb = K / 32;
     const uint16_t* xr = reinterpret_cast<const uint16_t*>(X) + ((size_t)t0 * nkb * 64 + lane) * 8;
     const uint16_t* wr = reinterpret_cast<const uint16_t*>(weights + woff) + ((size_t)(n0 / kBatchTile) * nkb * 64 + lane) * 8;
-    struct Frag {
-      u32x4_t w[CT], x[NT];
-    };
-    auto load = [&](int k, Frag& f) {
+    if constexpr (kCastNorm) {
+      // X is x in FP32 (16-column blocks): lane (r16, g) takes its eight columns as two 16-byte
+      // pieces and forms the FP16 operand (x . scale) . g, each value as batch_norm_mixed has it.
+      const float* xs = reinterpret_cast<const float*>(X) +
+                        (((size_t)t0 * 2 * nkb + (g >> 1)) * 64 + r16 + 32 * (g & 1)) * 4;
+      const uint16_t* gr = reinterpret_cast<const uint16_t*>(weights + w_norm);
+      // The slices' sums of squares: lane l loads rows 4 (l % 4) .. + 3 of column quad l / 4.
+      const float* sr = reinterpret_cast<const float*>(X) - kSquares + squares_index(t0 * kBatchTile, 0) + 4 * lane;
+      f4v part[SW][NT];
 #pragma unroll
-      for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
+      for (int i = 0; i < SW; i++)
 #pragma unroll
-      for (int t = 0; t < NT; t++) f.x[t] = gload16(xr + ((size_t)t * nkb + k / 32) * 512);
-    };
-    auto mma = [&](int i, const Frag& f) {
+        for (int t = 0; t < NT; t++) {
+          const float* p = sr + squares_index(t * kBatchTile, (first + i) * (slice / 4));
+          part[i][t] = gload16f(p);
+          // Slices are 64 or 128 columns: 16 or 32 quads.
+          if (slice > 64) part[i][t] += gload16f(p + 256);
+        }
+      asm volatile("" ::: "memory");
+      float scale[NT];
+      auto scales = [&] {
+        epsilon = ap->epsilon;
 #pragma unroll
-      for (int t = 0; t < NT; t++)
+        for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int c = 0; c < CT; c++)
-          acc[i][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, f.x[t]),
-                                                                __builtin_bit_cast(f16x8, f.w[c]), acc[i][t][c], 0, 0, 0);
-    };
-    auto pin = [&](Frag& f) {
+          for (int k = 0; k < 4; k++) {
+            float v = column_sum(part[0][t][k], 4);
+            if constexpr (SW == 2) v = v + column_sum(part[1][t][k], 4);
+            if (lane < 4) sq[wave][t][4 * lane + k] = v;
+          }
+        __syncthreads();
 #pragma unroll
-      for (int c = 0; c < CT; c++) pin4(f.w[c]);
+        for (int t = 0; t < NT; t++) scale[t] = 1.0f / sqrtf(tree([&](int k) { return sq[k][t][r16]; }) / (float)width + epsilon);
+      };
+      struct Frag {
+        u32x4_t w[CT], gn;
+        f4v xlo[NT], xhi[NT];
+      };
+      auto load = [&](int k, Frag& f) {
 #pragma unroll
-      for (int t = 0; t < NT; t++) pin4(f.x[t]);
-    };
-    k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, early);
+        for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
+        f.gn = gload16(gr + norm_at(k + 8 * g, 8));
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          const float* p = xs + ((size_t)t * nkb + k / 32) * 512;
+          f.xlo[t] = gload16f(p);
+          f.xhi[t] = gload16f(p + 64);
+        }
+      };
+      auto mma = [&](int i, const Frag& f) {
+        const f16x8 gh = __builtin_bit_cast(f16x8, f.gn);
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          f16x8 xh;
+#pragma unroll
+          for (int j = 0; j < 8; j++) xh[j] = (_Float16)((j < 4 ? f.xlo[t][j & 3] : f.xhi[t][j & 3]) * scale[t] * (float)gh[j]);
+#pragma unroll
+          for (int c = 0; c < CT; c++)
+            acc[i][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, __builtin_bit_cast(f16x8, f.w[c]), acc[i][t][c], 0, 0, 0);
+        }
+      };
+      auto pin = [&](Frag& f) {
+#pragma unroll
+        for (int c = 0; c < CT; c++) pin4(f.w[c]);
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          pin4(f.xlo[t]);
+          pin4(f.xhi[t]);
+        }
+        pin4(f.gn);
+      };
+      k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, [&] {
+        early();
+        scales();
+      });
+    } else {
+      struct Frag {
+        u32x4_t w[CT], x[NT];
+      };
+      auto load = [&](int k, Frag& f) {
+#pragma unroll
+        for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
+#pragma unroll
+        for (int t = 0; t < NT; t++) f.x[t] = gload16(xr + ((size_t)t * nkb + k / 32) * 512);
+      };
+      auto mma = [&](int i, const Frag& f) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+          for (int c = 0; c < CT; c++)
+            acc[i][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, f.x[t]),
+                                                                  __builtin_bit_cast(f16x8, f.w[c]), acc[i][t][c], 0, 0, 0);
+      };
+      auto pin = [&](Frag& f) {
+#pragma unroll
+        for (int c = 0; c < CT; c++) pin4(f.w[c]);
+#pragma unroll
+        for (int t = 0; t < NT; t++) pin4(f.x[t]);
+      };
+      k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, early);
+    }
   }
   // A wave holding two slices adds them here: the first level of the tree.
 #pragma unroll
@@ -489,19 +591,13 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
 #pragma unroll
       for (int r = 0; r < 4; r++) red[wave][t][c][4 * g + r][r16] = v[r];
     }
-    if constexpr (kNorm) {
+    if constexpr (kScale) {
       float v = column_sum(ss[0][t], 16);
       if constexpr (SW == 2) v = v + column_sum(ss[1][t], 16);
       if (g == 0) sq[wave][t][r16] = v;
     }
   }
   __syncthreads();
-  auto tree = [&](auto at) {
-    float p[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) p[k] = SW == 2 ? at(k) : at(2 * k) + at(2 * k + 1);
-    return (p[0] + p[1]) + (p[2] + p[3]);
-  };
 #pragma unroll
   for (int u = 0; u < kOwn; u++) {
     if (!owned(u)) break;
@@ -511,7 +607,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
     const int c = o.cc / kBatchTile, col = o.cc % kBatchTile;
     float s0 = tree([&](int k) { return red[k][o.t][c][o.row][col]; });
     float s1 = unit == 2 ? tree([&](int k) { return red[k][o.t][c][o.row][col + 1]; }) : 0.f;
-    if constexpr (kNorm) {
+    if constexpr (kScale) {
       const float sum = tree([&](int k) { return sq[k][o.t][o.row]; });
       const float scale = 1.0f / sqrtf(sum / (float)width + epsilon);
       s0 *= scale;
@@ -522,8 +618,16 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
     s0 = cast<P>(s0);
     s1 = cast<P>(s1);
     const int n = n0 + o.cc;
+    // Mixed mode: the squares of the four columns that a quad of lanes writes to x.
+    auto squares = [&](float v) {
+      if constexpr (P == kMixed) {
+        const float v2 = quad_squares(v);
+        if ((lane & 3) == 0) in_global(reinterpret_cast<float*>(out))[squares_index(b, n >> 2) - kSquares] = v2;
+      }
+    };
     if constexpr (E == kEpInput) {
       reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = s0;
+      squares(s0);
     } else if constexpr (E == kEpQkv) {
       // src/cuda/Primitives.cuh:148-166: RoPE on adjacent pairs of q and k, then the ring write.
       const int sec = (n >= width) + (n >= 2 * width);
@@ -549,7 +653,9 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         *in_global(reinterpret_cast<v2f*>(base + dst)) = v2f{va, vb};
       }
     } else if constexpr (E == kEpOut) {
-      reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = cast<P>(res[u] + s0);
+      const float v = cast<P>(res[u] + s0);
+      reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = v;
+      squares(v);
     } else if constexpr (E == kEpGateUp) {
       const float v = cast<P>((s0 / (1.0f + expf(-s0))) * s1);
       if constexpr (P == kMixed) reinterpret_cast<uint16_t*>(out)[half_index(b, n >> 1, out_ld)] = float_to_half(v);
@@ -557,6 +663,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
     } else {
       const float v = cast<P>(res[u] + s0);
       reinterpret_cast<float*>(out)[act_index<P>(b, n, out_ld)] = v;
+      squares(v);
       in_global(hidden)[((size_t)b * layers + layer) * width + n] = v;
     }
   }
@@ -963,42 +1070,44 @@ __device__ __forceinline__ float batch_weight(const char* w, uint32_t off, int i
   return bf16_to_float(reinterpret_cast<const uint16_t*>(w + off)[i]);
 }
 
-// Mixed mode: RMSNorm of every stream's x into xn with the output cast to FP16
-// (src/cuda/Primitives.cuh:122-135); padding columns and padding streams are zero. One
-// workgroup of 256 threads per row of the padded batch. Every load (x and the norm vector,
-// at most 4 columns per thread) is issued before the reduction, so the kernel waits one
-// memory round trip; the sums keep their order.
+// Mixed mode, batches whose projections do not fold the norm: RMSNorm of every stream's x into xn
+// with the output cast to FP16 (src/cuda/Primitives.cuh:122-135); padding columns and padding
+// streams are zero. One workgroup of 256 threads per row of the padded batch; a wave takes two of
+// the eight K-slices. The sum of squares is added as the writers of x and the folding projections
+// add it (column quads, a slice's 64-column pieces, slices), so that a stream's bits do not depend
+// on which of the two ran. Every load (x and the norm vector, at most 4 columns per thread) is
+// issued before the reduction: one memory round trip.
 static __global__ __launch_bounds__(256) void batch_norm_mixed(const BatchArgs* __restrict__ ap, uint32_t w_norm) {
   const BatchArgs& a = *ap;
   __shared__ float red[4];
-  const int b = blockIdx.x;
+  const int b = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float* x = a.x;
   uint16_t* out = reinterpret_cast<uint16_t*>(a.xn);
-  auto xb = [&](int i) { return x[act_index<kMixed>(b, i, a.width_p)]; };
   if (b >= a.streams) {
     for (int i = threadIdx.x; i < a.width_p; i += blockDim.x) out[half_index(b, i, a.width_p)] = 0;
     return;
   }
   constexpr int kPer = kMaxDim / 256;
-  float xv[kPer], gv[kPer];
+  const int per = a.width_p / 256;  // 64-column pieces of the wave: 2 (one per slice) or 4
+  float xv[kPer], gv[kPer], sq[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
-    const int i = threadIdx.x + 256 * j;
-    xv[j] = i < a.width ? xb(i) : 0.f;
-    gv[j] = i < a.width ? batch_weight<kMixed>(a.weights, w_norm, i) : 0.f;
+    const int i = (wave * per + j) * 64 + lane;
+    const bool in = j < per && i < a.width;
+    xv[j] = in ? x[act_index<kMixed>(b, i, a.width_p)] : 0.f;
+    gv[j] = in ? batch_weight<kMixed>(a.weights, w_norm, i) : 0.f;
   }
-  float s = 0.f;
 #pragma unroll
-  for (int j = 0; j < kPer; j++)
-    if (threadIdx.x + 256 * j < a.width) s += xv[j] * xv[j];
-  s = wave_total(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  for (int j = 0; j < kPer; j++) sq[j] = quad_squares(xv[j]);
+  const float s0 = per > 2 ? sq[0] + sq[1] : sq[0], s1 = per > 2 ? sq[2] + sq[3] : sq[1];
+  const float s = column_sum(s0, 4) + column_sum(s1, 4);
+  if (lane == 0) red[wave] = s;
   __syncthreads();
   const float scale = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)a.width + a.epsilon);
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
-    const int i = threadIdx.x + 256 * j;
-    if (i < a.width_p) out[half_index(b, i, a.width_p)] = i < a.width ? float_to_half(xv[j] * scale * gv[j]) : 0;
+    const int i = (wave * per + j) * 64 + lane;
+    if (j < per) out[half_index(b, i, a.width_p)] = i < a.width ? float_to_half(xv[j] * scale * gv[j]) : 0;
   }
 }
 

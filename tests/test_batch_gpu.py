@@ -160,6 +160,24 @@ def test_attention_chunks_match_a_batch_of_one_and_the_oracle(dim, heads, window
                 np.testing.assert_array_equal(x, y)
 
 
+@pytest.mark.parametrize('width,heads,streams', [(1024, 16, 70), (528, 11, 256)])
+def test_mixed_norm_kernels_match_folded_norms(width, heads, streams):
+    # At these sizes the batch's norms are kernels of their own; a batch of one folds them into its
+    # projections (528: padding columns in the last slices). Scores and state must agree bit for bit.
+    c = ModelConfig(2, width, heads, 256, 12, 40)
+    w = synthetic_checkpoint(c, seed=19, mixed=True)
+    events = _events(c, 19, 16, streams)
+    with batch((c, w, True), streams) as rt:
+        many = np.stack([rt.step(e) for e in events])
+        states = {b: rt.snapshot(b) for b in (0, streams - 1)}
+    for b, state in states.items():
+        with batch((c, w, True), 1) as one:
+            alone = np.array([one.step(e[b:b + 1])[0] for e in events], dtype=np.float32)
+            np.testing.assert_array_equal(alone, many[:, b])
+            for x, y in zip(one.snapshot(0), state):
+                np.testing.assert_array_equal(x, y)
+
+
 # head dim 128: attention rows of two 64-element pieces
 @pytest.mark.parametrize('name,streams,steps', [('main', 16, 40), ('small', 19, 90), ('dh128', 6, 60),
                                                 ('wide', 3, 48), ('odd', 5, 60)])
