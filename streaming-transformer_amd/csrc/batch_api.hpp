@@ -70,9 +70,9 @@ class Batch : public BatchBase {
   StreamHandle stream_;
   GraphHandle graph_;
   GraphExecHandle graph_exec_;
-  DeviceBuffer weights_, keys_, values_, hidden_, position_, in_, x_, xn_, attn_, act_, q_, score_, rope_, step_rope_, step_slot_,
+  DeviceBuffer weights_, keys_, values_, hidden_, position_, in_, x_, xn_, attn_, act_, q_, rope_, step_rope_, step_slot_,
       args_dev_, attn_part_, attn_count_;
-  PinnedBuffer host_in_, host_out_;
+  MappedBuffer host_in_, host_out_;
   StepArgs offsets_{};  // weight arena offsets (shared layout with the single-stream runtime)
   BatchArgs args_{};
   const BatchArgs* dargs_ = nullptr;

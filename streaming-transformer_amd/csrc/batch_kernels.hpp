@@ -46,7 +46,7 @@ struct BatchArgs {
   float* attn;                     // attention output (FP16 in mixed mode; width_p)
   float* act;                      // SwiGLU output (FP16 in mixed mode; ffn_p)
   float* q;                        // [Bp][width] rotated queries
-  float* score;                    // [B]
+  float* score;                    // [B], host memory mapped into the device
   float2* rope;                    // [Bp][dim / 2] cos, sin of this step's position (batch_proj, kEpInput)
   int* slot;                       // [Bp] ring slot of this step's position
 };
@@ -1136,6 +1136,28 @@ __global__ __launch_bounds__(64) void batch_final(const BatchArgs* __restrict__ 
     a.score[b] = acc;
     a.position[b] = a.position[b] + 1;
   }
+}
+
+// Rows row0 .. row0 + rows - 1 of a step's events, [streams][features] in host memory mapped into
+// the device, into the padded input block in the projections' operand layout. A thread per four
+// columns: a wave reads up to 1 KB contiguous across PCIe, every piece in one round trip.
+// Padding columns stay zero.
+template <int P>
+__global__ __launch_bounds__(256) void batch_stage(const float* __restrict__ events, float* __restrict__ in, int row0,
+                                                   int rows, int features, int features_p) {
+  const int per_row = (features + 3) / 4, i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i >= rows * per_row) return;
+  const int b = row0 + i / per_row, k = i % per_row * 4;
+  const float* src = events + (size_t)b * features + k;
+  f4v v = {0.f, 0.f, 0.f, 0.f};
+  if (features % 4 == 0) {
+    v = gload16f(src);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (k + j < features) v[j] = src[j];
+  }
+  *in_global(reinterpret_cast<f4v*>(in + act_index<P>(b, k, features_p))) = v;
 }
 
 // Zero the state of stream `stream` (every stream when negative): K/V rows, hidden, position.

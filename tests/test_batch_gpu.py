@@ -160,6 +160,22 @@ def test_attention_chunks_match_a_batch_of_one_and_the_oracle(dim, heads, window
                 np.testing.assert_array_equal(x, y)
 
 
+@pytest.mark.parametrize('features,streams', [(1021, 70), (1024, 33), (3, 2)])
+@pytest.mark.parametrize('weight_dtype', [WeightStorage.AS_MODEL, WeightStorage.BF16])
+def test_staged_events_match_a_batch_of_one(features, streams, weight_dtype):
+    # 70 and 33 streams of 4 KB events: staged in pieces of 32 streams, the last one partial; 1021
+    # and 3 features: rows that are not whole 16-byte pieces.
+    c = ModelConfig(1, 64, 2, 128, 16, features)
+    w = synthetic_checkpoint(c, seed=20)
+    events = _events(c, 20, 6, streams)
+    with batch((c, w, False), streams, weight_dtype) as rt:
+        many = np.stack([rt.step(e) for e in events])
+    for b in range(0, streams, max(1, streams // 7)):
+        with batch((c, w, False), 1, weight_dtype) as one:
+            alone = np.array([one.step(e[b:b + 1])[0] for e in events], dtype=np.float32)
+        np.testing.assert_array_equal(alone, many[:, b])
+
+
 @pytest.mark.parametrize('width,heads,streams', [(1024, 16, 70), (528, 11, 256)])
 def test_mixed_norm_kernels_match_folded_norms(width, heads, streams):
     # At these sizes the batch's norms are kernels of their own; a batch of one folds them into its
