@@ -29,12 +29,10 @@ Batch::Batch(const st_config& config, bool mixed, const st_tensor* tensors, size
     throw Error(ST_ERR_INVALID, "bfloat16 weight storage applies to FP32 checkpoints only");
   prec_ = mixed ? kMixed : weight_dtype == ST_WEIGHTS_BF16 ? kBf16w : kFp32;
   streams_ = streams;
-  // Padded batch: 16 or 32 rows, else a multiple of 64, so that every projection's batch
-  // groups (1, 2 or 4 tiles of 16) divide it.
+  // Padded batch: 16 or 32 rows, else a multiple of 64, so that a projection's batch groups (1 or 4
+  // tiles of 16) divide it.
   streams_p_ = streams <= 16 ? 16 : streams <= 32 ? 32 : (streams + 63) / 64 * 64;
   dim_ = c_.width / c_.heads;
-  wide_qkv_ = (3 * c_.width / kBatchTile) % 2 == 0;
-  wide_gateup_ = (2 * c_.ffn / kBatchTile) % 2 == 0;
   if (dim_ % 4) throw Error(ST_ERR_INVALID, "Batched streams need a head dimension that is a multiple of 4");
   int device = 0;
   HIP_CHECK(hipGetDevice(&device));
@@ -126,40 +124,38 @@ Batch::~Batch() {
   if (stream_) (void)hipStreamSynchronize(stream_);  // before the buffers are freed
 }
 
-// Batch tiles per projection workgroup: the largest of 4, 2, 1 that still gives at least 256
-// workgroups (one per CU), so that narrow projections at small batches spread over the chip.
-// `cols` is the number of column groups (N / (16 CT)); at most `max_tiles` batch tiles.
-int Batch::group_tiles(int cols, int max_tiles) const {
-  const int tiles = streams_p_ / kBatchTile;
-  for (int nt = std::min(kGroupTiles, max_tiles); nt > 1; nt >>= 1)
-    if (tiles % nt == 0 && cols * (tiles / nt) >= 256) return nt;
-  return 1;
-}
-
-template <int P, int E, bool kNorm, int CT, int SW>
-void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer,
-                    int max_tiles) {
-  const int cols = N / (kBatchTile * CT);
-  const int nt = group_tiles(cols, max_tiles);
-  const dim3 grid(cols, streams_p_ / kBatchTile / nt), block(64 * kSlices / SW);
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream_, args_.weights, X, out, dargs_, woff, ld, norm, c_.width, streams_,
-                       out_ld, layer);
-  };
-  // Blocks in flight per wave (k_ring): four where a slice holds a multiple of four and the
-  // workgroup has at most two tiles, else two.
+// One projection. Every workgroup shape computes the same fixed slice tree, so the choice changes
+// speed only, never a stream's bits. Each workgroup re-reads its rows of X and its rows of the
+// weights, and converts X to MFMA operands, so more column tiles (CT) share both; the chip wants
+// about as many workgroups as it has CUs. So CT is the largest of 4, 2, 1 that leaves kWorkgroups,
+// with one batch tile (NT): us per layer against two K-slices per wave and 1 to 4 batch tiles, the
+// shapes of before, gate/up 4 x 1 -3.1 for Large at 32 streams, -12.2 at 128, -0.8 for Main at 64;
+// QKV 2 x 1 -1.2 for Large at 32, 4 x 1 -4.4 at 128; narrow projections of small models (128 tiles)
+// 1 x 1 instead of 2 x 1 -1.3 for Small at 100. At one batch tile a wider CT gains nothing (Large
+// at 8 streams, gate/up 2 x 1 +0.1 to +0.5).
+// Mixed mode's norm kernels hand over X in FP16: nothing to convert, and weights are most of the
+// traffic, so four batch tiles share them (2 x 4: Large at 128 streams, QKV -1.1 and gate/up -3.4
+// against 4 x 1; at 256 -1.0 and -2.4).
+template <int P, int E, bool kNorm>
+void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer) {
+  const int cols = N / kBatchTile, batch_tiles = streams_p_ / kBatchTile;
+  // Blocks in flight per wave (k_ring): four where a slice holds a multiple of four, else two.
   constexpr int kb = P == kFp32 || (P == kMixed && E == kEpInput) ? 16 : 32;
   const bool deep = ld / kSlices / kb % 4 == 0;
-  auto ring = [&](auto NT) {
-    constexpr int nt_ = decltype(NT)::value;
-    if constexpr (SW == 1 && nt_ * CT <= 2) {
-      if (deep) return go(batch_proj<P, E, kNorm, nt_, CT, SW, 4>);
-    }
-    go(batch_proj<P, E, kNorm, nt_, CT, SW, 2>);
+  auto go = [&](auto kernel, int nt, int ct) {
+    hipLaunchKernelGGL(kernel, dim3(cols / ct, batch_tiles / nt), dim3(64 * kSlices), 0, stream_, args_.weights, X, out,
+                       dargs_, woff, ld, norm, c_.width, streams_, out_ld, layer);
   };
-  if (nt == 4) ring(std::integral_constant<int, 4>{});
-  else if (nt == 2) ring(std::integral_constant<int, 2>{});
-  else ring(std::integral_constant<int, 1>{});
+  auto fits = [&](int ct) { return batch_tiles > 1 && cols % ct == 0 && cols / ct * batch_tiles >= kWorkgroups; };
+  if constexpr (P == kMixed && !kNorm && (E == kEpQkv || E == kEpGateUp)) {
+    if (cols % 2 == 0 && batch_tiles % 4 == 0) return go(batch_proj<P, E, kNorm, 4, 2, 2>, 4, 2);
+  }
+  if constexpr (E != kEpInput) {
+    if (fits(4)) return go(batch_proj<P, E, kNorm, 1, 4, 2>, 1, 4);
+    if (fits(2)) return deep ? go(batch_proj<P, E, kNorm, 1, 2, 4>, 1, 2) : go(batch_proj<P, E, kNorm, 1, 2, 2>, 1, 2);
+  }
+  if (deep) go(batch_proj<P, E, kNorm, 1, 1, 4>, 1, 1);
+  else go(batch_proj<P, E, kNorm, 1, 1, 2>, 1, 1);
 }
 
 // Attention of one layer. Windows of more than one chunk: a workgroup per (stream, head, chunk)
@@ -207,22 +203,10 @@ void Batch::attend(int layer) {
   }
 }
 
-// Workgroup shapes per projection. Every shape computes the same fixed slice tree, so the
-// choice changes speed only, never a stream's bits. Small batches want many workgroups (one
-// column tile and one K-slice per wave); large ones want each X fragment reused across column
-// tiles: from 64 streams the wide projections (QKV, gate/up) take two column tiles and two
-// K-slices per wave, and from 128 streams the narrow ones (OUT, down) take two column tiles.
-// From 256 streams (16-bit operands), gate/up takes four column tiles and one K-slice per
-// wave (eight waves), and QKV one batch tile per workgroup: measured on Main at 256 streams,
-// gate/up 15.2 -> 12.5 us and QKV 11.6 -> 10.0 us per layer with bfloat16 weights
-// (9.3 -> 8.0 and 8.5 -> 7.5 us in mixed mode), from fewer re-reads of X across column tiles
-// and more workgroups respectively.
 template <int P>
 void Batch::launch_sequence() {
   const BatchArgs& a = args_;
   const int d = c_.width, F = c_.ffn;
-  const bool wide = streams_p_ >= 64, narrow = streams_p_ >= 128 && (c_.width / kBatchTile) % 2 == 0;
-  const bool huge = P != kFp32 && streams_p_ >= 256;
   // K/V rings that do not fit in the Infinity Cache beside the weights are read with
   // non-temporal loads, so that the weights stay cached.
   const bool kv_nt = 2 * c_.layers * (size_t)streams_ * block_words_ * 4 + offsets_.weight_bytes > kInfinityCacheBytes;
@@ -238,39 +222,29 @@ void Batch::launch_sequence() {
   auto norm = [&](uint32_t w_norm) {
     if (!fold) hipLaunchKernelGGL(batch_norm_mixed, dim3(streams_p_), dim3(256), 0, stream_, dargs_, w_norm);
   };
-  auto qkv_gateup = [&](const LayerWeights& w, int l, auto kFold, auto qkv) {
-    constexpr bool kf = decltype(kFold)::value;
-    if constexpr (decltype(qkv)::value) {
-      if (wide && wide_qkv_)
-        project<P, kEpQkv, kf, 2, 2>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l, huge ? 1 : kGroupTiles);
-      else project<P, kEpQkv, kf, 1, 1>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
-    } else {
-      if (huge && (2 * F / kBatchTile) % 4 == 0)
-        project<P, kEpGateUp, kf, 4, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
-      else if (wide && wide_gateup_)
-        project<P, kEpGateUp, kf, 2, 2>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
-      else project<P, kEpGateUp, kf, 1, 1>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
-    }
+  auto qkv = [&](const LayerWeights& w, int l, auto kFold) {
+    project<P, kEpQkv, decltype(kFold)::value>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
   };
-  auto normed = [&](const LayerWeights& w, int l, auto qkv) {
+  auto gateup = [&](const LayerWeights& w, int l, auto kFold) {
+    project<P, kEpGateUp, decltype(kFold)::value>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
+  };
+  auto normed = [&](auto&& projection, const LayerWeights& w, int l) {
     if constexpr (P == kMixed) {
-      if (!fold) return qkv_gateup(w, l, std::false_type{}, qkv);
+      if (!fold) return projection(w, l, std::false_type{});
     }
-    qkv_gateup(w, l, std::true_type{}, qkv);
+    projection(w, l, std::true_type{});
   };
-  project<P, kEpInput, false, 1, 1>(a.in, a.features_p, a.x, a.width_p, a.w_input, d, 0u, 0);
+  project<P, kEpInput, false>(a.in, a.features_p, a.x, a.width_p, a.w_input, d, 0u, 0);
   for (int l = 0; l < c_.layers; l++) {
     const LayerWeights& w = a.layer[l];
     norm(w.norm1);
-    normed(w, l, std::true_type{});
+    normed(qkv, w, l);
     if (kv_nt) attend<P, true>(l);
     else attend<P, false>(l);
-    if (narrow) project<P, kEpOut, false, 2, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
-    else project<P, kEpOut, false, 1, 1>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
+    project<P, kEpOut, false>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
     norm(w.norm2);
-    normed(w, l, std::false_type{});
-    if (narrow) project<P, kEpDown, false, 2, 1>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
-    else project<P, kEpDown, false, 1, 1>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
+    normed(gateup, w, l);
+    project<P, kEpDown, false>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
   }
   hipLaunchKernelGGL(batch_final<P>, dim3(streams_), dim3(64), 0, stream_, dargs_);
   HIP_CHECK(hipGetLastError());

@@ -51,12 +51,10 @@ class Batch : public BatchBase {
     const int chunks = attn_chunks();
     return dim_ <= 128 && chunks > 1 && (chunks > kAttnLoop || streams_ * c_.heads < kSplitPairs);
   }
-  template <int P, int E, bool kNorm, int CT, int SW>
-  void project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer,
-               int max_tiles = kGroupTiles);
-  int group_tiles(int cols, int max_tiles) const;
+  template <int P, int E, bool kNorm>
+  void project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer);
+  static constexpr int kWorkgroups = 192;  // fewest workgroups of a projection with wider tiles (project)
   void stage_events(const float* inputs, float* block) const;
-  bool wide_qkv_ = false, wide_gateup_ = false;  // two column tiles per workgroup
   size_t block_words_ = 0;  // one (layer, stream) block [H][W][dh] of the K (or V) ring, in 4-byte words
   void launch() {
     if (prec_ == kFp32) launch_sequence<kFp32>();

@@ -115,7 +115,6 @@ __host__ __device__ __forceinline__ size_t half_index(int b, int n, int cols) {
   const int kk = n & 31;
   return (((size_t)(b >> 4) * (cols >> 5) + (n >> 5)) * 64 + (b & 15) + 16 * (kk >> 3)) * 8 + (kk & 7);
 }
-constexpr int kGroupTiles = 4;   // most batch tiles (16 streams each) per projection workgroup
 
 enum BatchEpilogue : int { kEpInput = 0, kEpQkv, kEpOut, kEpGateUp, kEpDown };
 
@@ -143,11 +142,11 @@ __device__ __forceinline__ void split3(const float (&x)[8], unsigned (&ph)[4], u
   }
 }
 
-// The K loop of one wave over its SW slices, from slice `first`, in blocks of KB columns: a ring
-// of R steps (a step is one block of each slice), unrolled so that no fragment is copied: step
-// j + R is loaded into the fragments of step j as soon as step j's MFMAs are issued, so R steps
-// are in flight while one computes. The host picks R = 4 for one-slice waves of at most two
-// tiles when the slice holds a multiple of 4 blocks (it always holds an even number), else 2.
+// The K loop of one wave over its slice, columns k0 .. k0 + slice - 1, in blocks of KB columns: a
+// ring of R blocks, unrolled so that no fragment is copied: block j + R is loaded into the
+// fragments of block j as soon as block j's MFMAs are issued, so R blocks are in flight while one
+// computes. The host picks R = 4 for workgroups of at most two tiles when the slice holds a
+// multiple of 4 blocks (it always holds an even number), else 2.
 // Three things hold the schedule: an empty asm after each prefetch (the compiler would otherwise
 // see that the loads only feed the next round and move them next to their use); `pin`, which
 // passes a fragment's registers through an asm right before its MFMAs (the compiler would
@@ -156,38 +155,31 @@ __device__ __forceinline__ void split3(const float (&x)[8], unsigned (&ph)[4], u
 // (pinned as scalars, the loop carried a register copy per element, which waited for every
 // load at the end of each round: Large with bfloat16 weights at 32 streams 645 -> 595 us per step).
 // `early` runs once, when the first R steps' loads are in flight: the epilogue's own operands
-// are fetched there, so that their round trips overlap the loop's. Every form issues a slice's
+// are fetched there, so that their round trips overlap the loop's. Every form issues the
 // MFMAs in block order.
-template <int R, int SW, int KB, typename Frag, typename Load, typename Pin, typename Mma, typename Early>
-__device__ __forceinline__ void k_ring(int first, int slice, Load&& load, Pin&& pin, Mma&& mma, Early&& early) {
+template <int R, int KB, typename Frag, typename Load, typename Pin, typename Mma, typename Early>
+__device__ __forceinline__ void k_ring(int k0, int slice, Load&& load, Pin&& pin, Mma&& mma, Early&& early) {
   const int nb = slice / KB;
-  Frag f[R][SW];
+  Frag f[R];
 #pragma unroll
-  for (int r = 0; r < R; r++)
-#pragma unroll
-    for (int i = 0; i < SW; i++) load((first + i) * slice + r * KB, f[r][i]);
+  for (int r = 0; r < R; r++) load(k0 + r * KB, f[r]);
   asm volatile("" ::: "memory");
   early();
   int j = 0;
   for (; j + R < nb; j += R) {
 #pragma unroll
     for (int r = 0; r < R; r++) {
-#pragma unroll
-      for (int i = 0; i < SW; i++) {
-        pin(f[r][i]);
-        mma(i, f[r][i]);
-        load((first + i) * slice + (j + R + r) * KB, f[r][i]);
-      }
+      pin(f[r]);
+      mma(f[r]);
+      load(k0 + (j + R + r) * KB, f[r]);
       asm volatile("" ::: "memory");
     }
   }
 #pragma unroll
-  for (int r = 0; r < R; r++)
-#pragma unroll
-    for (int i = 0; i < SW; i++) {
-      pin(f[r][i]);
-      mma(i, f[r][i]);
-    }
+  for (int r = 0; r < R; r++) {
+    pin(f[r]);
+    mma(f[r]);
+  }
 }
 
 __device__ __forceinline__ void pin4(u32x4_t& v) { asm volatile("" : "+v"(v)); }
@@ -195,13 +187,12 @@ __device__ __forceinline__ void pin4(f4v& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin4(u32x2_t& v) { asm volatile("" : "+v"(v)); }
 
 // One projection Y = X . W^T over the batch, with its phase's epilogue. Workgroup: CT column
-// tiles of 16 outputs and NT batch tiles of 16 streams. K is cut into 8 slices; each wave
-// accumulates SW of them (8 / SW waves) for every tile pair with MFMA, reusing each X
-// fragment for the CT column tiles and each weight fragment for the NT batch tiles. The slice
-// partials are added in one fixed pairwise tree, ((s0 + s1) + (s2 + s3)) + ((s4 + s5) +
-// (s6 + s7)), whatever NT, CT and SW are, so a stream's outputs depend only on its own row
-// and are bit-identical for every batch size. The padded batch is a multiple of NT tiles, so
-// the loops have no branches. X and W are in the tiled operand layout (act_index and the tiled
+// tiles of 16 outputs and NT batch tiles of 16 streams. K is cut into 8 slices; each of the 8 waves
+// accumulates one for every tile pair with MFMA, reusing each X fragment for the CT column tiles
+// and each weight fragment for the NT batch tiles. The slice partials are added in one fixed
+// pairwise tree, ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)), whatever NT and CT are, so a
+// stream's outputs depend only on its own row and are bit-identical for every batch size. The
+// padded batch is a multiple of NT tiles, so the loops have no branches. X and W are in the tiled operand layout (act_index and the tiled
 // arena): one 16 x KB block of either is 64 lanes' contiguous 16-byte pieces in lane order.
 // X is the padded buffer of K columns; W the N x K matrix at offset `woff` of the arena
 // `weights`; `out` the phase's output buffer (row length out_ld): x, or the SwiGLU output.
@@ -226,13 +217,13 @@ __device__ __forceinline__ void pin4(u32x2_t& v) { asm volatile("" : "+v"(v)); }
 // the ring geometry) is fetched while the K loop's first loads are in flight: read after the
 // loop, each of those was a dependent memory round trip on a kernel of 3-5 us (Main with
 // bfloat16 weights at 16 streams 195 -> 188 us per step, Large at 32 streams 595 -> 576 us).
-template <int P, int E, bool kNorm, int NT, int CT, int SW, int R>
-__global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __restrict__ weights,
-                                                               const void* __restrict__ X, void* out,
-                                                               const BatchArgs* __restrict__ ap, uint32_t woff, int K,
-                                                               uint32_t w_norm, int width, int streams, int out_ld,
-                                                               int layer) {
-  constexpr int kWaves = kSlices / SW, kBlock = 64 * kWaves;
+template <int P, int E, bool kNorm, int NT, int CT, int R>
+__global__ __launch_bounds__(64 * kSlices) void batch_proj(const char* __restrict__ weights,
+                                                           const void* __restrict__ X, void* out,
+                                                           const BatchArgs* __restrict__ ap, uint32_t woff, int K,
+                                                           uint32_t w_norm, int width, int streams, int out_ld,
+                                                           int layer) {
+  constexpr int kWaves = kSlices, kBlock = 64 * kWaves;
   constexpr bool kCastNorm = kNorm && P == kMixed;  // the norm's output is cast before the MFMAs
   constexpr bool kScale = kNorm && P != kMixed;     // the epilogue applies the norm's scale
   const BatchArgs& a = *ap;
@@ -242,8 +233,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
   const int n0 = blockIdx.x * kBatchTile * CT;
   const int t0 = blockIdx.y * NT;
   const int r16 = lane & 15, g = lane >> 4;
-  const int slice = K / kSlices;
-  const int first = wave * SW;  // the wave's first slice
+  const int slice = K / kSlices, k0 = wave * slice;
 
   // Epilogue units of this thread: a column, or the column pair of a RoPE or gate-up pair, of
   // one stream. Unit u of the workgroup's tiles is, for the phases that write an activation
@@ -324,21 +314,19 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
       }
     }
   };
-  f4v acc[SW][NT][CT];
-  float ss[SW][NT];
+  f4v acc[NT][CT];
+  float ss[NT];
 #pragma unroll
-  for (int i = 0; i < SW; i++)
+  for (int t = 0; t < NT; t++) {
+    ss[t] = 0.f;
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-      ss[i][t] = 0.f;
-#pragma unroll
-      for (int c = 0; c < CT; c++) acc[i][t][c] = f4v{0.f, 0.f, 0.f, 0.f};
-    }
-  // The slices' fixed tree over the waves' partials (their pairs already added where SW is 2).
+    for (int c = 0; c < CT; c++) acc[t][c] = f4v{0.f, 0.f, 0.f, 0.f};
+  }
+  // The slices' fixed tree over the waves' partials.
   auto tree = [&](auto at) {
     float p[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) p[k] = SW == 2 ? at(k) : at(2 * k) + at(2 * k + 1);
+    for (int k = 0; k < 4; k++) p[k] = at(2 * k) + at(2 * k + 1);
     return (p[0] + p[1]) + (p[2] + p[3]);
   };
   // Index of the norm weights of columns k .. k + n - 1. The vector holds `width` values (a
@@ -372,15 +360,15 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
 #pragma unroll
       for (int t = 0; t < NT; t++) f.x[t] = gload16f(xr + ((size_t)t * nkb + k / 16) * 256);
     };
-    auto mma = [&](int i, const Frag& f) {
+    auto mma = [&](const Frag& f) {
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         f4v x = f.x[t];
         if constexpr (kNorm) {
-          ss[i][t] += x.x * x.x;
-          ss[i][t] += x.y * x.y;
-          ss[i][t] += x.z * x.z;
-          ss[i][t] += x.w * x.w;
+          ss[t] += x.x * x.x;
+          ss[t] += x.y * x.y;
+          ss[t] += x.z * x.z;
+          ss[t] += x.w * x.w;
           x.x *= f.gn.x;
           x.y *= f.gn.y;
           x.z *= f.gn.z;
@@ -388,7 +376,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         }
 #pragma unroll
         for (int c = 0; c < CT; c++) {
-          f4v& d = acc[i][t][c];
+          f4v& d = acc[t][c];
           d = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, f.w[c].x, d, 0, 0, 0);
           d = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, f.w[c].y, d, 0, 0, 0);
           d = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, f.w[c].z, d, 0, 0, 0);
@@ -403,7 +391,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
       for (int t = 0; t < NT; t++) pin4(f.x[t]);
       if constexpr (kNorm) pin4(f.gn);
     };
-    k_ring<R, SW, 16, Frag>(first, slice, load, pin, mma, early);
+    k_ring<R, 16, Frag>(k0, slice, load, pin, mma, early);
   } else if constexpr (P == kBf16w) {
     // Tiled operands: weight block (tile, k / 32) holds 64 lanes x 8 values, activation block
     // two planes of 64 lanes x 4 floats.
@@ -426,7 +414,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         f.xhi[t] = gload16f(p + 256);
       }
     };
-    auto mma = [&](int i, const Frag& f) {
+    auto mma = [&](const Frag& f) {
       float gv[8];
       if constexpr (kNorm) {
         const unsigned gu[4] = {f.gn.x, f.gn.y, f.gn.z, f.gn.w};
@@ -442,7 +430,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         if constexpr (kNorm) {
 #pragma unroll
           for (int j = 0; j < 8; j++) {
-            ss[i][t] += x[j] * x[j];
+            ss[t] += x[j] * x[j];
             x[j] *= gv[j];
           }
         }
@@ -453,7 +441,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
 #pragma unroll
         for (int c = 0; c < CT; c++) {
           const bf16x8 wb = __builtin_bit_cast(bf16x8, f.w[c]);
-          f4v& d = acc[i][t][c];
+          f4v& d = acc[t][c];
           d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, wb, d, 0, 0, 0);
           d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m, wb, d, 0, 0, 0);
           d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, wb, d, 0, 0, 0);
@@ -470,7 +458,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
       }
       if constexpr (kNorm) pin4(f.gn);
     };
-    k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, early);
+    k_ring<R, 32, Frag>(k0, slice, load, pin, mma, early);
   } else {
     // Mixed mode: the operand is an FP16 buffer (its values are cast points) and the weights
     // are FP16; one v_mfma_f32_16x16x32_f16 per 32-k block, lane (r16, g) holding
@@ -485,18 +473,16 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
       const float* xs = reinterpret_cast<const float*>(X) +
                         (((size_t)t0 * 2 * nkb + (g >> 1)) * 64 + r16 + 32 * (g & 1)) * 4;
       const uint16_t* gr = reinterpret_cast<const uint16_t*>(weights + w_norm);
-      // The slices' sums of squares: lane l loads rows 4 (l % 4) .. + 3 of column quad l / 4.
+      // The slice's sums of squares: lane l loads rows 4 (l % 4) .. + 3 of column quad l / 4.
       const float* sr = reinterpret_cast<const float*>(X) - kSquares + squares_index(t0 * kBatchTile, 0) + 4 * lane;
-      f4v part[SW][NT];
+      f4v part[NT];
 #pragma unroll
-      for (int i = 0; i < SW; i++)
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-          const float* p = sr + squares_index(t * kBatchTile, (first + i) * (slice / 4));
-          part[i][t] = gload16f(p);
-          // Slices are 64 or 128 columns: 16 or 32 quads.
-          if (slice > 64) part[i][t] += gload16f(p + 256);
-        }
+      for (int t = 0; t < NT; t++) {
+        const float* p = sr + squares_index(t * kBatchTile, k0 / 4);
+        part[t] = gload16f(p);
+        // Slices are 64 or 128 columns: 16 or 32 quads.
+        if (slice > 64) part[t] += gload16f(p + 256);
+      }
       asm volatile("" ::: "memory");
       float scale[NT];
       auto scales = [&] {
@@ -505,8 +491,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         for (int t = 0; t < NT; t++)
 #pragma unroll
           for (int k = 0; k < 4; k++) {
-            float v = column_sum(part[0][t][k], 4);
-            if constexpr (SW == 2) v = v + column_sum(part[1][t][k], 4);
+            const float v = column_sum(part[t][k], 4);
             if (lane < 4) sq[wave][t][4 * lane + k] = v;
           }
         __syncthreads();
@@ -528,7 +513,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
           f.xhi[t] = gload16f(p + 64);
         }
       };
-      auto mma = [&](int i, const Frag& f) {
+      auto mma = [&](const Frag& f) {
         const f16x8 gh = __builtin_bit_cast(f16x8, f.gn);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -537,7 +522,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
           for (int j = 0; j < 8; j++) xh[j] = (_Float16)((j < 4 ? f.xlo[t][j & 3] : f.xhi[t][j & 3]) * scale[t] * (float)gh[j]);
 #pragma unroll
           for (int c = 0; c < CT; c++)
-            acc[i][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, __builtin_bit_cast(f16x8, f.w[c]), acc[i][t][c], 0, 0, 0);
+            acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, __builtin_bit_cast(f16x8, f.w[c]), acc[t][c], 0, 0, 0);
         }
       };
       auto pin = [&](Frag& f) {
@@ -550,7 +535,7 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
         }
         pin4(f.gn);
       };
-      k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, [&] {
+      k_ring<R, 32, Frag>(k0, slice, load, pin, mma, [&] {
         early();
         scales();
       });
@@ -564,13 +549,13 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
 #pragma unroll
         for (int t = 0; t < NT; t++) f.x[t] = gload16(xr + ((size_t)t * nkb + k / 32) * 512);
       };
-      auto mma = [&](int i, const Frag& f) {
+      auto mma = [&](const Frag& f) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
           for (int c = 0; c < CT; c++)
-            acc[i][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, f.x[t]),
-                                                                  __builtin_bit_cast(f16x8, f.w[c]), acc[i][t][c], 0, 0, 0);
+            acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, f.x[t]),
+                                                                  __builtin_bit_cast(f16x8, f.w[c]), acc[t][c], 0, 0, 0);
       };
       auto pin = [&](Frag& f) {
 #pragma unroll
@@ -578,22 +563,17 @@ __global__ __launch_bounds__(64 * kSlices / SW) void batch_proj(const char* __re
 #pragma unroll
         for (int t = 0; t < NT; t++) pin4(f.x[t]);
       };
-      k_ring<R, SW, 32, Frag>(first, slice, load, pin, mma, early);
+      k_ring<R, 32, Frag>(k0, slice, load, pin, mma, early);
     }
   }
-  // A wave holding two slices adds them here: the first level of the tree.
 #pragma unroll
   for (int t = 0; t < NT; t++) {
 #pragma unroll
-    for (int c = 0; c < CT; c++) {
-      f4v v = acc[0][t][c];
-      if constexpr (SW == 2) v = acc[0][t][c] + acc[1][t][c];
+    for (int c = 0; c < CT; c++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) red[wave][t][c][4 * g + r][r16] = v[r];
-    }
+      for (int r = 0; r < 4; r++) red[wave][t][c][4 * g + r][r16] = acc[t][c][r];
     if constexpr (kScale) {
-      float v = column_sum(ss[0][t], 16);
-      if constexpr (SW == 2) v = v + column_sum(ss[1][t], 16);
+      const float v = column_sum(ss[t], 16);
       if (g == 0) sq[wave][t][r16] = v;
     }
   }
