@@ -1,6 +1,6 @@
 // The batched runtimes' interface (st_batch): BatchBase, and Batch, the graph of phase kernels
 // over B independent streams sharing one weight arena. A step is a fixed sequence of 5L + 2
-// kernels captured once in a hipGraph: the input projection, then per layer QKV (RMSNorm
+// kernels (two more per layer in mixed mode's large batches) captured once in a hipGraph: the input projection, then per layer QKV (RMSNorm
 // prologue, RoPE and ring-write epilogue), attention, OUT (+residual), gate/up (RMSNorm
 // prologue, SwiGLU epilogue), down (+residual, hidden), then the final norm and the scores.
 // Batch's members are defined in batch.hip, a translation unit of their own; the resident

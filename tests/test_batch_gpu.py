@@ -103,8 +103,7 @@ def test_bf16_weights_match_oracle_on_rounded_weights(name, streams, steps):
     (WeightStorage.AS_MODEL, False, 40, 70), (WeightStorage.BF16, False, 40, 70), (WeightStorage.AS_MODEL, True, 40, 70),
     # 130 streams: the large-batch workgroup shapes of every projection
     (WeightStorage.BF16, False, 130, 20), (WeightStorage.AS_MODEL, True, 130, 20),
-    # 256 streams: mixed mode's attention takes four passes of loads (against eight passes with
-    # V loaded early for a batch of one), past the window
+    # 256 streams: attention loads wait for the position (a batch of one's do not), past the window
     (WeightStorage.AS_MODEL, True, 256, 70)])
 def test_stream_independent_of_batch(weight_dtype, mixed, streams, steps):
     c = SHAPES['small']
@@ -268,7 +267,7 @@ def test_reset_one_and_all_and_device_run_equals_stepping():
                                              (WeightStorage.AS_MODEL, 64)])
 def test_large_rings_read_non_temporally_match_a_batch_of_one(weights, streams):
     # Main with FP32 K/V: from 64 streams the K/V rings and the weights exceed the Infinity
-    # Cache, and attention reads K/V with non-temporal loads (and other loop forms); a batch of
+    # Cache, and attention reads K/V with non-temporal loads; a batch of
     # one reads them with ordinary loads. Scores and state must agree bit for bit.
     c = SHAPES['main']
     w = synthetic_checkpoint(c, seed=17)
