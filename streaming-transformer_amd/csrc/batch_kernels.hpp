@@ -329,10 +329,9 @@ __global__ __launch_bounds__(64 * kSlices) void batch_proj(const char* __restric
     for (int k = 0; k < 4; k++) p[k] = at(2 * k) + at(2 * k + 1);
     return (p[0] + p[1]) + (p[2] + p[3]);
   };
-  // Index of the norm weights of columns k .. k + n - 1. The vector holds `width` values (a
-  // multiple of 16); padding columns, whose x is zero, take its last ones, so that the load has
-  // no branch around it (one in the K loop's rounds drained every load in flight).
-  auto norm_at = [&](int k, int n) { return k + n <= width ? k : width - n; };
+  // The arena pads a layer norm's gains with zeros to the K columns, so that their load has no
+  // branch around it (one in the K loop's rounds drained every load in flight) and a padding
+  // column's product is zero whatever the gains are.
   if constexpr (P == kFp32 || (P == kMixed && E == kEpInput)) {
     // FP32 MFMA. Mixed mode takes this path for the input projection only: its operand is
     // the raw FP32 event, and its FP16 weights widen exactly.
@@ -356,7 +355,7 @@ __global__ __launch_bounds__(64 * kSlices) void batch_proj(const char* __restric
                        half_to_float((unsigned short)(h.y & 0xffffu)), half_to_float((unsigned short)(h.y >> 16))};
         }
       }
-      if constexpr (kNorm) f.gn = gload16f(gr + norm_at(k + 4 * g, 4));
+      if constexpr (kNorm) f.gn = gload16f(gr + k + 4 * g);
 #pragma unroll
       for (int t = 0; t < NT; t++) f.x[t] = gload16f(xr + ((size_t)t * nkb + k / 16) * 256);
     };
@@ -406,7 +405,7 @@ __global__ __launch_bounds__(64 * kSlices) void batch_proj(const char* __restric
     auto load = [&](int k, Frag& f) {
 #pragma unroll
       for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
-      if constexpr (kNorm) f.gn = gload16(gr + norm_at(k + 8 * g, 8));
+      if constexpr (kNorm) f.gn = gload16(gr + k + 8 * g);
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const float* p = xr + ((size_t)t * nkb + k / 32) * 512;
@@ -505,7 +504,7 @@ __global__ __launch_bounds__(64 * kSlices) void batch_proj(const char* __restric
       auto load = [&](int k, Frag& f) {
 #pragma unroll
         for (int c = 0; c < CT; c++) f.w[c] = gload16(wr + ((size_t)c * nkb + k / 32) * 512);
-        f.gn = gload16(gr + norm_at(k + 8 * g, 8));
+        f.gn = gload16(gr + k + 8 * g);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
           const float* p = xs + ((size_t)t * nkb + k / 32) * 512;

@@ -632,6 +632,12 @@ void build_arena(const st_config& c_, int prec_, const st_tensor* tensors, size_
   auto put_vector = [&](const float* data, int n) {
     for (int i = 0; i < n; i++) put(data[i]);
   };
+  // A layer norm's gains, zero over the padding columns of the projections that fold the norm.
+  auto put_gains = [&](const float* data, int n, int cols_p) {
+    put_vector(data, n);
+    if (tiled)
+      for (int i = n; i < cols_p; i++) put(0.f);
+  };
   StepArgs& a = args_;
   const int d = c_.width, f = c_.ffn;
   align();
@@ -642,10 +648,10 @@ void build_arena(const st_config& c_, int prec_, const st_tensor* tensors, size_
     LayerWeights& lw = a.layer[l];
     align();
     lw.norm1 = (uint32_t)host.size();
-    put_vector(get(p + "norm1", {d})->data, d);
+    put_gains(get(p + "norm1", {d})->data, d, a.width_p);
     align();
     lw.norm2 = (uint32_t)host.size();
-    put_vector(get(p + "norm2", {d})->data, d);
+    put_gains(get(p + "norm2", {d})->data, d, a.width_p);
     align();
     lw.qkv = (uint32_t)host.size();
     {

@@ -193,6 +193,27 @@ def test_mixed_norm_kernels_match_folded_norms(width, heads, streams):
                 np.testing.assert_array_equal(x, y)
 
 
+@pytest.mark.parametrize('mixed', [False, True])
+def test_an_infinite_last_gain_stays_in_its_column(mixed):
+    # 96 columns of 256 (512 in mixed mode): the padding behind an infinite last gain adds nothing, so
+    # V, which is not rotated, is infinite with the sign of x and its weight, as in the oracle.
+    c = SHAPES['dh48']
+    w = synthetic_checkpoint(c, seed=21, mixed=mixed)
+    w['layers.0.norm1'][-1] = np.inf
+    events = _events(c, 21, 3, 2)
+    with batch((c, w, mixed), 2) as rt:
+        for e in events:
+            rt.step(e)
+        got = [rt.snapshot(b)[2][0] for b in range(2)]
+    for b in range(2):
+        oracle = Oracle(c, w, mixed=mixed, accumulate='double')
+        for e in events:
+            oracle.step(e[b])
+        want = oracle.snapshot()[2][0]
+        assert np.isinf(want[:, :3]).all()
+        np.testing.assert_array_equal(got[b], want)
+
+
 # head dim 128: attention rows of two 64-element pieces
 @pytest.mark.parametrize('name,streams,steps', [('main', 16, 40), ('small', 19, 90), ('dh128', 6, 60),
                                                 ('wide', 3, 48), ('odd', 5, 60)])
