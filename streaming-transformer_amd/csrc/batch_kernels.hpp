@@ -693,6 +693,13 @@ constexpr int kAttnWaves = kAttnThreads / 64;
 constexpr int kBatchChunk = 128;    // ring slots per attention chunk
 constexpr int kAttnLoop = 8;       // most chunks that one workgroup walks (its partials are in LDS)
 
+// The values of lanes 0 .. N - 1 of each row of 16 lanes, in every lane of the row.
+template <int N, int K = 0>
+__device__ __forceinline__ void row_values(float v, float (&out)[N]) {
+  out[K] = dpp_get<0x150 + K>(v);  // row_newbcast:K
+  if constexpr (K + 1 < N) row_values<N, K + 1>(v, out);
+}
+
 // Weight of a softmax partial with maximum m beside the overall maximum `top`. A partial without
 // finite logits (m = -inf) carries zeros and gets weight zero; if every logit is -inf the sum is
 // zero and the output 0 / 0, as a softmax over them has it.
@@ -720,6 +727,13 @@ __device__ __forceinline__ void put_attn(void* attn, int b, int n, int width_p, 
 // block, then the position, then K; a maximum, a sum and an output through LDS with five
 // barriers. Main with bfloat16 weights at 16 streams 188.7 -> 178.4 us per step, at 256 430.6 ->
 // 425.5; mixed mode at 64 streams 243.2 -> 239.3.)
+//
+// From a few hundred (stream, head) pairs of small heads or short rows on, the instructions bound
+// the kernel and not the loads: a row's division and exponential are computed by one of its 16
+// lanes and broadcast, chunks before the last test no slot, and empty half chunks are skipped (one
+// in each lane, every slot tested, no skip: mixed mode with 35 heads of 16, W = 282, 115 streams
+// 44.2 -> 30.3 us per layer; a step of three layers with 112 heads of 4, W = 409, 50 streams
+// 286 -> 205 us; Main at 16 streams 152.6 -> 150.7, bit-identical).
 //
 // Workgroups: gridDim.z == 1: one walks all chunks of its (stream, head), its partials in LDS.
 // Otherwise workgroup z takes chunk z, writes the chunk's partial through to memory and counts
@@ -789,9 +803,15 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned l
   // its own load.
   auto chunk = [&](int c, auto more) {
     const int c0 = c * kBatchChunk;
-    float lg[NP], mx = -INFINITY;
+    // Chunks before the last hold valid slots only.
+    auto live = [&](int pass) { return more.value || c0 + 16 * pass + grp < valid; };
+    // No valid slot in the last chunk's second half: its passes are skipped.
+    const bool both = more.value || c0 + 8 * NP < valid;
+    // Lane r keeps the logit of pass r mod NP, for one division and one exponential per row.
+    float lg = 0.f;
 #pragma unroll
     for (int p = 0; p < NP; p++) {
+      if (p >= NP / 2 && !both) break;
       float dot = 0.f;
 #pragma unroll
       for (int j = 0; j < DV; j++) {
@@ -804,31 +824,30 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned l
         dot = d + 64 * j < dim ? part_dot : dot;
       }
       dot = group_sum(dot, 16);
-      float l = dot / div;
-      asm volatile("" : "+v"(l));  // no branch around the division
-      lg[p] = c0 + 16 * p + grp < valid ? l : -INFINITY;
-      mx = fmaxf(mx, lg[p]);
+      lg = r % NP == p ? dot : lg;
     }
     if constexpr (more.value) load(keys, kv, c0 + kBatchChunk, valid);
-    mx = wave_top(mx);
+    lg = live(r % NP) ? lg / div : -INFINITY;
+    const float mx = wave_top(lg);
     const float ref = mx == -INFINITY ? 0.f : mx;
+    float e[NP];
+    row_values<NP>(expf(lg - ref), e);
     float sum = 0.f;
     f4v o[DV];
 #pragma unroll
     for (int j = 0; j < DV; j++) o[j] = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-      const float e = expf(lg[p] - ref);
-      sum += e;
-      const bool live = c0 + 16 * p + grp < valid;
+      if (p >= NP / 2 && !both) break;
+      sum += e[p];
 #pragma unroll
       for (int j = 0; j < DV; j++) {
         pin4(vv[p][j]);
         const f4v v = widen(vv[p][j]);
-        o[j].x = live ? __builtin_fmaf(e, v.x, o[j].x) : o[j].x;
-        o[j].y = live ? __builtin_fmaf(e, v.y, o[j].y) : o[j].y;
-        o[j].z = live ? __builtin_fmaf(e, v.z, o[j].z) : o[j].z;
-        o[j].w = live ? __builtin_fmaf(e, v.w, o[j].w) : o[j].w;
+        o[j].x = live(p) ? __builtin_fmaf(e[p], v.x, o[j].x) : o[j].x;
+        o[j].y = live(p) ? __builtin_fmaf(e[p], v.y, o[j].y) : o[j].y;
+        o[j].z = live(p) ? __builtin_fmaf(e[p], v.z, o[j].z) : o[j].z;
+        o[j].w = live(p) ? __builtin_fmaf(e[p], v.w, o[j].w) : o[j].w;
       }
     }
     if constexpr (more.value) load(values, vv, c0 + kBatchChunk, valid);

@@ -129,6 +129,8 @@ def test_stream_independent_of_batch(weight_dtype, mixed, streams, steps):
     (48, 4, 128, 70, 133, True),    # a full chunk, lanes past the head dim
     (64, 4, 129, 66, 135, False),   # two chunks, the second of one slot
     (48, 4, 300, 65, 310, True),    # three chunks
+    (12, 4, 192, 70, 200, False),   # a last chunk of exactly its first half
+    (4, 16, 193, 40, 200, True),    # and of one slot more
     (128, 2, 200, 130, 210, False),  # two pieces of 64 elements per row
     (68, 4, 130, 64, 133, True),    # the second piece of four elements
     (160, 2, 140, 3, 145, False),   # the wide form
