@@ -159,11 +159,12 @@ void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff,
 }
 
 // Attention of one layer. Windows of more than one chunk: a workgroup per (stream, head, chunk)
-// where the (stream, head) pairs alone give fewer than kSplitPairs workgroups, one per CU (or the
-// window has more chunks than one workgroup keeps), else one that walks its chunks. Split, Main
-// with W = 1024 at 4 streams (32 pairs) went 249 -> 199 us per step; above the line a merge costs
-// more than the spread gives: 296 pairs of two chunks 111.8 us walked, 114.2 split; Large at 32
-// streams (512 pairs of four) 574 walked, 586 split.
+// where the (stream, head) pairs alone give fewer than kSplitPairs workgroups, else one that walks
+// its chunks. Below the line the spread fills the chip: us per step of two layers, split / walked,
+// at 32 pairs 52.8 / 60.7 (FP16 K/V, eight chunks) and 80.2 / 97.7 (FP32, 16 chunks, head dim 128),
+// at 128 pairs 60.5 / 62.7 and 142.9 / 144.2. From the line on the partials written, counted and
+// read back cost more than that gives: at 192 pairs 64.0 / 64.5 and 187.6 / 169.7, with 32 chunks
+// 216.0 / 170.3 (FP32, head dim 64), at 512 pairs of 16 chunks 236 / 205.
 template <int P, bool kNT>
 void Batch::attend(int layer) {
   const size_t block = (size_t)c_.width * c_.window * (P == kMixed ? 2 : 4);  // a (layer, stream) block in bytes
@@ -185,7 +186,7 @@ void Batch::attend(int layer) {
   // The loads that do not wait for the position read every slot of the window: for one-chunk
   // windows whose rings stay cached and that are too few to fill the chip (elsewhere the unwritten
   // slots' bytes would cost more than the round trip).
-  const bool any = !kNT && chunks == 1 && streams_ * c_.heads <= kSplitPairs;
+  const bool any = !kNT && chunks == 1 && streams_ * c_.heads <= kAnyPairs;
   auto form = [&](auto DV, auto NP) {
     constexpr int dv = decltype(DV)::value, np = decltype(NP)::value;
     if constexpr (!kNT) {

@@ -45,11 +45,12 @@ class Batch : public BatchBase {
   template <int P> void launch_sequence();
   template <int P, bool kNT> void attend(int layer);
   // Chunks of the attention window, and whether they are spread over workgroups (batch_attention).
-  static constexpr int kSplitPairs = 256;
+  static constexpr int kSplitPairs = 192;  // fewest (stream, head) pairs whose workgroups walk them (attend)
+  static constexpr int kAnyPairs = 256;    // most pairs that leave the chip with room for unwritten slots
   int attn_chunks() const { return (c_.window + kBatchChunk - 1) / kBatchChunk; }
   bool attn_split() const {
     const int chunks = attn_chunks();
-    return dim_ <= 128 && chunks > 1 && (chunks > kAttnLoop || streams_ * c_.heads < kSplitPairs);
+    return dim_ <= 128 && chunks > 1 && streams_ * c_.heads < kSplitPairs;
   }
   template <int P, int E, bool kNorm>
   void project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer);

@@ -691,7 +691,6 @@ __device__ __forceinline__ f4v widen(u32x2_t h) {
 constexpr int kAttnThreads = 256;  // batch_attention's workgroup: four waves, 16 groups of 16 lanes
 constexpr int kAttnWaves = kAttnThreads / 64;
 constexpr int kBatchChunk = 128;    // ring slots per attention chunk
-constexpr int kAttnLoop = 8;       // most chunks that one workgroup walks (its partials are in LDS)
 
 // The values of lanes 0 .. N - 1 of each row of 16 lanes, in every lane of the row.
 template <int N, int K = 0>
@@ -721,8 +720,8 @@ __device__ __forceinline__ void put_attn(void* attn, int b, int n, int width_p, 
 // each, so a wave's load covers 4 rows; a wave owns 4 rows of each of the NP passes of 16 rows,
 // and the chunk's K and V loads are all issued before the first dot product (NP = 8; windows of
 // at most 64 slots take NP = 4). Each wave forms its own softmax partial of a chunk: its rows'
-// maximum m, s = sum exp(l - m), o = sum exp(l - m) V, in registers. One barrier, then wave 0 merges
-// the four waves' partials of each chunk, and the chunks in order. So the critical path of a
+// maximum m, s = sum exp(l - m), o = sum exp(l - m) V, in registers. One barrier, then the
+// four waves' partials of each chunk are merged, and the chunks in order. So the critical path of a
 // one-chunk window is: position, K and V in one round trip, one barrier. (Before: the arguments
 // block, then the position, then K; a maximum, a sum and an output through LDS with five
 // barriers. Main with bfloat16 weights at 16 streams 188.7 -> 178.4 us per step, at 256 430.6 ->
@@ -735,7 +734,9 @@ __device__ __forceinline__ void put_attn(void* attn, int b, int n, int width_p, 
 // 44.2 -> 30.3 us per layer; a step of three layers with 112 heads of 4, W = 409, 50 streams
 // 286 -> 205 us; Main at 16 streams 152.6 -> 150.7, bit-identical).
 //
-// Workgroups: gridDim.z == 1: one walks all chunks of its (stream, head), its partials in LDS.
+// Workgroups: gridDim.z == 1: one walks all chunks of its (stream, head), its partials in LDS (at most
+// 32 chunks: 34 KB for head dims up to 64, else 67 KB, where registers hold a CU to two to four
+// workgroups anyway).
 // Otherwise workgroup z takes chunk z, writes the chunk's partial through to memory and counts
 // itself; the last to arrive merges the chunks (it finds every partial there: nothing waits).
 // Both run the same arithmetic in the same order, so a stream's bits do not depend on the form,
@@ -875,7 +876,6 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned l
   for (; c + 1 < last; c++) chunk(c, std::true_type{});
   chunk(c, std::false_type{});
   __syncthreads();
-  if (wave != 0) return;
   // The merges, each lane for its own columns lane + 64 j. No FMA contraction: both forms must
   // round alike.
   auto merge_waves = [&](int c, float& m, float& s, float (&o)[DV]) {
@@ -900,11 +900,6 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned l
       if (lane + 64 * j < dim) put_attn<P>(attn, b, h * dim + lane + 64 * j, width_p, num[j] / den);
   };
   float m, s, o[DV];
-  if (active == 1) {
-    merge_waves(0, m, s, o);
-    put(o, s);
-    return;
-  }
   float num[DV], den = 0.f, top = -INFINITY;
 #pragma unroll
   for (int j = 0; j < DV; j++) num[j] = 0.f;
@@ -915,13 +910,38 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned l
 #pragma unroll
     for (int j = 0; j < DV; j++) num[j] = num[j] + oc[j] * e;
   };
-  if (!split) {
-    for (int k = 0; k < active * kAttnWaves; k++) top = fmaxf(top, part[k * kRow + 64 * DV]);
-    for (int c = 0; c < active; c++) {
+  if (!split && active > 1) {
+    // A wave merges every fourth chunk, into the place of the chunk's first partial; wave 0 adds the
+    // chunks in order. (One wave merging all: 512 pairs of 32 chunks 363.8 -> 358.7 us per step of
+    // two layers, of 16 FP16 chunks at 1024 pairs 210.6 -> 204.3.)
+    auto row = [&](int c) { return part + c * kAttnWaves * kRow; };
+    for (int c = wave; c < active; c += kAttnWaves) {
       merge_waves(c, m, s, o);
-      add_chunk(m, s, o);
+      float* to = row(c);
+#pragma unroll
+      for (int j = 0; j < DV; j++) to[lane + 64 * j] = o[j];
+      if (lane == 0) {
+        to[64 * DV] = m;
+        to[64 * DV + 1] = s;
+      }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    for (int c = lane; c < active; c += 64) top = fmaxf(top, row(c)[64 * DV]);
+    top = wave_top(top);
+#pragma unroll 4
+    for (int c = 0; c < active; c++) {
+#pragma unroll
+      for (int j = 0; j < DV; j++) o[j] = row(c)[lane + 64 * j];
+      add_chunk(row(c)[64 * DV], row(c)[64 * DV + 1], o);
     }
     put(num, den);
+    return;
+  }
+  if (wave != 0) return;
+  if (active == 1) {
+    merge_waves(0, m, s, o);
+    put(o, s);
     return;
   }
   // This chunk's partial, written through to memory (agent scope) and complete before the count.
@@ -944,8 +964,8 @@ __global__ __launch_bounds__(kAttnThreads) void batch_attention(const unsigned l
   asm volatile("" ::: "memory");
   if (lane == 0) __hip_atomic_store(arrived + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   auto get = [&](int c, int i) { return __hip_atomic_load(at(c, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  // Up to kAttnLoop chunks in one round trip, any others (windows over 1024 slots) after it.
-  constexpr int kAhead = kAttnLoop;
+  // Up to kAhead chunks in one round trip, any others (windows over 1024 slots) after it.
+  constexpr int kAhead = 8;
   float mc[kAhead], sc[kAhead], oc[kAhead][DV];
 #pragma unroll
   for (int c = 0; c < kAhead; c++) {
