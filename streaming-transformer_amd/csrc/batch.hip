@@ -124,6 +124,30 @@ Batch::~Batch() {
   if (stream_) (void)hipStreamSynchronize(stream_);  // before the buffers are freed
 }
 
+// Column tiles of a projection's workgroup with one batch tile (project).
+int Batch::column_tiles(int cols) const {
+  const int batch_tiles = streams_p_ / kBatchTile;
+  for (int ct = 4; ct > 1; ct >>= 1)
+    if (batch_tiles > 1 && cols % ct == 0 && cols / ct * batch_tiles >= kWorkgroups) return ct;
+  return 1;
+}
+
+// Mixed mode: whether a projection of `cols` column tiles folds its norm. Folded, it saves the norm's
+// kernel and converts its X rows again in each group of column tiles; behind the norm's kernel it
+// takes X in FP16, four batch tiles to a workgroup. So it folds where there are no four tiles, else up
+// to kFoldWork values converted: rows x K x groups. us per layer of the fold against the norm's kernel,
+// swept over widths 256 to 1024, ffn 256 to 4096 and 1 to 256 streams: up to 32 streams always
+// less (-1.1 to -2.6). From 64 on, gate/up at 4.2 M -3.9 to -1.3, 8.4 M -0.6 to -0.1, 12.6 M -0.3 to
+// +1.1, 16.8 M +2.8 and +3.4; QKV at 6.3 M -1.4 and -1.2, 9.4 M -0.1 to +0.4, 12.6 M -0.1 and +0.3. Odd
+// column tile counts, whose four-tile shape shares X with no second column tile: 11.3 M -0.8, 12.3 M
+// +0.6, 14.2 M +0.3, 16.7 M +2.1. (One width, 528, whose groups fall on the XCDs unevenly, loses 1 us at
+// 4.3 M.)
+bool Batch::folds_norm(int cols) const {
+  const size_t line = (size_t)(cols % 2 ? 12 : 8) << 20;
+  return streams_p_ % (4 * kBatchTile) != 0 ||
+         (size_t)streams_p_ * args_.width_p * (cols / column_tiles(cols)) <= line;
+}
+
 // One projection. Every workgroup shape computes the same fixed slice tree, so the choice changes
 // speed only, never a stream's bits. Each workgroup re-reads its rows of X and its rows of the
 // weights, and converts X to MFMA operands, so more column tiles (CT) share both; the chip wants
@@ -135,7 +159,8 @@ Batch::~Batch() {
 // at 8 streams, gate/up 2 x 1 +0.1 to +0.5).
 // Mixed mode's norm kernels hand over X in FP16: nothing to convert, and weights are most of the
 // traffic, so four batch tiles share them (2 x 4: Large at 128 streams, QKV -1.1 and gate/up -3.4
-// against 4 x 1; at 256 -1.0 and -2.4).
+// against 4 x 1; at 256 -1.0 and -2.4; odd column tile counts 1 x 4: 173 of gate/up at 192 streams
+// -3.4 against 1 x 1, 105 of QKV at 128 -2.1).
 template <int P, int E, bool kNorm>
 void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer) {
   const int cols = N / kBatchTile, batch_tiles = streams_p_ / kBatchTile;
@@ -146,16 +171,18 @@ void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff,
     hipLaunchKernelGGL(kernel, dim3(cols / ct, batch_tiles / nt), dim3(64 * kSlices), 0, stream_, args_.weights, X, out,
                        dargs_, woff, ld, norm, c_.width, streams_, out_ld, layer);
   };
-  auto fits = [&](int ct) { return batch_tiles > 1 && cols % ct == 0 && cols / ct * batch_tiles >= kWorkgroups; };
   if constexpr (P == kMixed && !kNorm && (E == kEpQkv || E == kEpGateUp)) {
-    if (cols % 2 == 0 && batch_tiles % 4 == 0) return go(batch_proj<P, E, kNorm, 4, 2, 2>, 4, 2);
+    if (cols % 2 == 0) go(batch_proj<P, E, kNorm, 4, 2, 2>, 4, 2);
+    else go(batch_proj<P, E, kNorm, 4, 1, 2>, 4, 1);
+  } else {
+    const int ct = E == kEpInput ? 1 : column_tiles(cols);
+    if constexpr (E != kEpInput) {
+      if (ct == 4) return go(batch_proj<P, E, kNorm, 1, 4, 2>, 1, 4);
+      if (ct == 2) return deep ? go(batch_proj<P, E, kNorm, 1, 2, 4>, 1, 2) : go(batch_proj<P, E, kNorm, 1, 2, 2>, 1, 2);
+    }
+    if (deep) go(batch_proj<P, E, kNorm, 1, 1, 4>, 1, 1);
+    else go(batch_proj<P, E, kNorm, 1, 1, 2>, 1, 1);
   }
-  if constexpr (E != kEpInput) {
-    if (fits(4)) return go(batch_proj<P, E, kNorm, 1, 4, 2>, 1, 4);
-    if (fits(2)) return deep ? go(batch_proj<P, E, kNorm, 1, 2, 4>, 1, 2) : go(batch_proj<P, E, kNorm, 1, 2, 2>, 1, 2);
-  }
-  if (deep) go(batch_proj<P, E, kNorm, 1, 1, 4>, 1, 1);
-  else go(batch_proj<P, E, kNorm, 1, 1, 2>, 1, 1);
 }
 
 // Attention of one layer. Windows of more than one chunk: a workgroup per (stream, head, chunk)
@@ -211,40 +238,33 @@ void Batch::launch_sequence() {
   // K/V rings that do not fit in the Infinity Cache beside the weights are read with
   // non-temporal loads, so that the weights stay cached.
   const bool kv_nt = 2 * c_.layers * (size_t)streams_ * block_words_ * 4 + offsets_.weight_bytes > kInfinityCacheBytes;
-  // The norms are folded into the projections (kNorm). Mixed mode casts a norm's output, so a
-  // folding projection converts its X rows (streams x K) again for each of its column tiles (N,
-  // like K the width times a constant); past kFoldWork of them the norms run first, into xn.
-  // Main steps without the fold and with it: 167.7 -> 142.9 us at one stream, 177 -> 144 at 16,
-  // 200 -> 177 at 64, 251 -> 246 at 128, 321 -> 315 at 256; four layers of Large: 134.5 -> 115.5 at
-  // 8, 171.1 -> 171.5 at 32, 221 -> 223 at 64, 325 -> 363 at 128.
-  constexpr size_t kFoldWork = (size_t)256 * 512 * 512;
-  const bool fold = P != kMixed || (size_t)streams_p_ * c_.width * c_.width <= kFoldWork;
-  const void* nx = fold ? a.x : a.xn;
-  auto norm = [&](uint32_t w_norm) {
-    if (!fold) hipLaunchKernelGGL(batch_norm_mixed, dim3(streams_p_), dim3(256), 0, stream_, dargs_, w_norm);
+  // The norms are folded into the projections (kNorm), or run first, into xn. Main's mixed steps
+  // without the fold and with it: 167.7 -> 142.9 us at one stream, 177 -> 144 at 16, 200 -> 177 at 64.
+  const bool fold_qkv = P != kMixed || folds_norm(3 * d / kBatchTile);
+  const bool fold_gateup = P != kMixed || folds_norm(2 * F / kBatchTile);
+  auto qkv = [&](const LayerWeights& w, int l, const void* x, auto kFold) {
+    project<P, kEpQkv, decltype(kFold)::value>(x, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
   };
-  auto qkv = [&](const LayerWeights& w, int l, auto kFold) {
-    project<P, kEpQkv, decltype(kFold)::value>(nx, a.width_p, nullptr, 0, w.qkv, 3 * d, w.norm1, l);
+  auto gateup = [&](const LayerWeights& w, int l, const void* x, auto kFold) {
+    project<P, kEpGateUp, decltype(kFold)::value>(x, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
   };
-  auto gateup = [&](const LayerWeights& w, int l, auto kFold) {
-    project<P, kEpGateUp, decltype(kFold)::value>(nx, a.width_p, a.act, a.ffn_p, w.gateup, 2 * F, w.norm2, l);
-  };
-  auto normed = [&](auto&& projection, const LayerWeights& w, int l) {
+  auto normed = [&](auto&& projection, const LayerWeights& w, uint32_t w_norm, int l, bool fold) {
     if constexpr (P == kMixed) {
-      if (!fold) return projection(w, l, std::false_type{});
+      if (!fold) {
+        hipLaunchKernelGGL(batch_norm_mixed, dim3(streams_p_), dim3(256), 0, stream_, dargs_, w_norm);
+        return projection(w, l, a.xn, std::false_type{});
+      }
     }
-    projection(w, l, std::true_type{});
+    projection(w, l, a.x, std::true_type{});
   };
   project<P, kEpInput, false>(a.in, a.features_p, a.x, a.width_p, a.w_input, d, 0u, 0);
   for (int l = 0; l < c_.layers; l++) {
     const LayerWeights& w = a.layer[l];
-    norm(w.norm1);
-    normed(qkv, w, l);
+    normed(qkv, w, w.norm1, l, fold_qkv);
     if (kv_nt) attend<P, true>(l);
     else attend<P, false>(l);
     project<P, kEpOut, false>(a.attn, a.width_p, a.x, a.width_p, w.out, d, 0u, l);
-    norm(w.norm2);
-    normed(gateup, w, l);
+    normed(gateup, w, w.norm2, l, fold_gateup);
     project<P, kEpDown, false>(a.act, a.ffn_p, a.x, a.width_p, w.down, d, 0u, l);
   }
   hipLaunchKernelGGL(batch_final<P>, dim3(streams_), dim3(64), 0, stream_, dargs_);

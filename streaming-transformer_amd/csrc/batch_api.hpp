@@ -1,6 +1,6 @@
 // The batched runtimes' interface (st_batch): BatchBase, and Batch, the graph of phase kernels
 // over B independent streams sharing one weight arena. A step is a fixed sequence of 5L + 2
-// kernels (two more per layer in mixed mode's large batches) captured once in a hipGraph: the input projection, then per layer QKV (RMSNorm
+// kernels (up to two more per layer in mixed mode's large batches) captured once in a hipGraph: the input projection, then per layer QKV (RMSNorm
 // prologue, RoPE and ring-write epilogue), attention, OUT (+residual), gate/up (RMSNorm
 // prologue, SwiGLU epilogue), down (+residual, hidden), then the final norm and the scores.
 // Batch's members are defined in batch.hip, a translation unit of their own; the resident
@@ -52,6 +52,8 @@ class Batch : public BatchBase {
     const int chunks = attn_chunks();
     return dim_ <= 128 && chunks > 1 && streams_ * c_.heads < kSplitPairs;
   }
+  int column_tiles(int cols) const;
+  bool folds_norm(int cols) const;
   template <int P, int E, bool kNorm>
   void project(const void* X, int ld, void* out, int out_ld, uint32_t woff, int N, uint32_t norm, int layer);
   static constexpr int kWorkgroups = 192;  // fewest workgroups of a projection with wider tiles (project)

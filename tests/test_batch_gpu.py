@@ -179,11 +179,16 @@ def test_staged_events_match_a_batch_of_one(features, streams, weight_dtype):
         np.testing.assert_array_equal(alone, many[:, b])
 
 
-@pytest.mark.parametrize('width,heads,streams', [(1024, 16, 70), (528, 11, 256)])
-def test_mixed_norm_kernels_match_folded_norms(width, heads, streams):
-    # At these sizes the batch's norms are kernels of their own; a batch of one folds them into its
+@pytest.mark.parametrize('width,heads,ffn,streams', [
+    (1024, 16, 256, 70),   # both folded, four column tiles and one
+    (528, 11, 256, 256),   # QKV's a kernel of its own (odd column tiles), gate/up's folded
+    (1024, 16, 4096, 130),  # both kernels of their own, two column tiles
+    (528, 11, 1000, 256),  # both, odd column tiles
+])
+def test_mixed_norm_kernels_match_folded_norms(width, heads, ffn, streams):
+    # At these sizes norms of the batch are kernels of their own; a batch of one folds them into its
     # projections (528: padding columns in the last slices). Scores and state must agree bit for bit.
-    c = ModelConfig(2, width, heads, 256, 12, 40)
+    c = ModelConfig(2, width, heads, ffn, 12, 40)
     w = synthetic_checkpoint(c, seed=19, mixed=True)
     events = _events(c, 19, 16, streams)
     with batch((c, w, True), streams) as rt:
