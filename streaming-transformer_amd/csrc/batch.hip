@@ -191,7 +191,10 @@ void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff,
 // at 32 pairs 52.8 / 60.7 (FP16 K/V, eight chunks) and 80.2 / 97.7 (FP32, 16 chunks, head dim 128),
 // at 128 pairs 60.5 / 62.7 and 142.9 / 144.2. From the line on the partials written, counted and
 // read back cost more than that gives: at 192 pairs 64.0 / 64.5 and 187.6 / 169.7, with 32 chunks
-// 216.0 / 170.3 (FP32, head dim 64), at 512 pairs of 16 chunks 236 / 205.
+// 216.0 / 170.3 (FP32, head dim 64), at 512 pairs of 16 chunks 236 / 205. A few pairs more than one
+// per CU put two walks on a few CUs, which the others wait for: at 264 pairs 68.8 / 75.5 (FP16, eight
+// chunks), 95.8 / 104.1 and 150.3 / 160.8 (FP32, eight and 16); even at 320, 72.8 / 76.4, 106.3 / 107.7 and
+// 169.7 / 166.5.
 template <int P, bool kNT>
 void Batch::attend(int layer) {
   const size_t block = (size_t)c_.width * c_.window * (P == kMixed ? 2 : 4);  // a (layer, stream) block in bytes
@@ -213,7 +216,7 @@ void Batch::attend(int layer) {
   // The loads that do not wait for the position read every slot of the window: for one-chunk
   // windows whose rings stay cached and that are too few to fill the chip (elsewhere the unwritten
   // slots' bytes would cost more than the round trip).
-  const bool any = !kNT && chunks == 1 && streams_ * c_.heads <= kAnyPairs;
+  const bool any = !kNT && chunks == 1 && streams_ * c_.heads <= kCuPairs;
   auto form = [&](auto DV, auto NP) {
     constexpr int dv = decltype(DV)::value, np = decltype(NP)::value;
     if constexpr (!kNT) {

@@ -135,12 +135,17 @@ def test_stream_independent_of_batch(weight_dtype, mixed, streams, steps):
     (68, 4, 130, 64, 133, True),    # the second piece of four elements
     (160, 2, 140, 3, 145, False),   # the wide form
     (32, 2, 1040, 130, 1050, False),  # nine chunks: more than a merge of a split window reads at once
+    # 320 pairs: walked (between 256 and 320 they are split, as below 192)
+    (64, 4, 129, 80, 135, False),
+    (48, 4, 300, 80, 310, True),
+    (128, 2, 200, 160, 210, False),
+    (32, 2, 1040, 160, 1050, False),
     (128, 2, 4096, 96, 1300, False),  # partials of 32 chunks in LDS, eleven of them written; non-temporal K/V
     (64, 16, 4096, 8, 140, False),    # split over workgroups with non-temporal K/V
 ])
 def test_attention_chunks_match_a_batch_of_one_and_the_oracle(dim, heads, window, streams, steps, mixed):
-    # A batch of one spreads a window's chunks over workgroups; at 192 or more (stream, head)
-    # pairs one workgroup walks them. Both must give the same bits, before and after the ring wraps.
+    # A batch of one spreads a window's chunks over workgroups; at most sizes from 192 (stream, head)
+    # pairs on one workgroup walks them. Both must give the same bits, before and after the ring wraps.
     c = ModelConfig(1, dim * heads, heads, 64, window, 24)
     w = synthetic_checkpoint(c, seed=18, mixed=mixed)
     events = _events(c, 18, steps, streams)
