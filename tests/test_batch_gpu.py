@@ -101,7 +101,7 @@ def test_bf16_weights_match_oracle_on_rounded_weights(name, streams, steps):
 
 @pytest.mark.parametrize('weight_dtype,mixed,streams,steps', [
     (WeightStorage.AS_MODEL, False, 40, 70), (WeightStorage.BF16, False, 40, 70), (WeightStorage.AS_MODEL, True, 40, 70),
-    # 130 streams: the large-batch workgroup shapes of every projection
+    # 130 streams (192 rows): two column tiles per workgroup in QKV, four in gate/up, one in OUT and down
     (WeightStorage.BF16, False, 130, 20), (WeightStorage.AS_MODEL, True, 130, 20),
     # 256 streams: attention loads wait for the position (a batch of one's do not), past the window
     (WeightStorage.AS_MODEL, True, 256, 70)])
@@ -121,6 +121,34 @@ def test_stream_independent_of_batch(weight_dtype, mixed, streams, steps):
         assert ref[0] == state[0]
         for x, y in zip(ref[1:], state[1:]):
             np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize('weights,mixed,width,ffn,streams', [
+    (WeightStorage.AS_MODEL, False, 1024, 4096, 130),  # four column tiles in every projection
+    (WeightStorage.BF16, False, 1024, 4096, 130),
+    (WeightStorage.AS_MODEL, True, 1024, 4096, 130),   # the same in OUT and down
+    (WeightStorage.AS_MODEL, False, 512, 2048, 130),   # two in OUT and down
+    (WeightStorage.BF16, False, 512, 2048, 130),
+    (WeightStorage.AS_MODEL, True, 512, 2048, 130),
+    (WeightStorage.AS_MODEL, True, 1024, 4096, 20),    # folded norms of 1024 columns: two tiles in QKV,
+    (WeightStorage.AS_MODEL, True, 1024, 4096, 64),    # then four; four in gate/up
+    (WeightStorage.AS_MODEL, True, 528, 1000, 33),     # odd column tiles: one each
+])
+def test_projection_shapes_equal_a_batch_of_one(weights, mixed, width, ffn, streams):
+    # A batch of one runs every projection with one column tile and one batch tile.
+    c = ModelConfig(2, width, width // 16, ffn, 8, 40)
+    w = synthetic_checkpoint(c, seed=22, mixed=mixed)
+    events = _events(c, 22, 10, streams)
+    picks = (0, streams // 2, streams - 1)
+    with batch((c, w, mixed), streams, weights) as rt:
+        many = np.stack([rt.step(e) for e in events])
+        states = [rt.snapshot(b) for b in picks]
+    for b, state in zip(picks, states):
+        with batch((c, w, mixed), 1, weights) as one:
+            alone = np.array([one.step(e[b:b + 1])[0] for e in events], dtype=np.float32)
+            np.testing.assert_array_equal(alone, many[:, b])
+            for x, y in zip(one.snapshot(0)[1:], state[1:]):
+                np.testing.assert_array_equal(x, y)
 
 
 @pytest.mark.parametrize('dim,heads,window,streams,steps,mixed', [
