@@ -194,7 +194,8 @@ void Batch::project(const void* X, int ld, void* out, int out_ld, uint32_t woff,
 // 216.0 / 170.3 (FP32, head dim 64), at 512 pairs of 16 chunks 236 / 205. A few pairs more than one
 // per CU put two walks on a few CUs, which the others wait for: at 264 pairs 68.8 / 75.5 (FP16, eight
 // chunks), 95.8 / 104.1 and 150.3 / 160.8 (FP32, eight and 16); even at 320, 72.8 / 76.4, 106.3 / 107.7 and
-// 169.7 / 166.5.
+// 169.7 / 166.5. Two chunks are walked there too (62.6 / 62.0, head dim 128 75.3 / 73.9; three 67.0 / 68.1
+// and 87.9 / 89.7).
 template <int P, bool kNT>
 void Batch::attend(int layer) {
   const size_t block = (size_t)c_.width * c_.window * (P == kMixed ? 2 : 4);  // a (layer, stream) block in bytes

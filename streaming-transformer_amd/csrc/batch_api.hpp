@@ -45,12 +45,14 @@ class Batch : public BatchBase {
   template <int P> void launch_sequence();
   template <int P, bool kNT> void attend(int layer);
   // Chunks of the attention window, and whether they are spread over workgroups (batch_attention).
-  // (stream, head) pairs: fewer than kSplitPairs, or one per CU and fewer than kSpillPairs, are split (attend).
+  // (stream, head) pairs whose chunks are split: fewer than kSplitPairs, or, of three chunks or more, between
+  // one per CU and kSpillPairs (attend).
   static constexpr int kSplitPairs = 192, kCuPairs = 256, kSpillPairs = 320;
   int attn_chunks() const { return (c_.window + kBatchChunk - 1) / kBatchChunk; }
   bool attn_split() const {
-    const int pairs = streams_ * c_.heads;
-    return dim_ <= 128 && attn_chunks() > 1 && (pairs < kSplitPairs || (pairs > kCuPairs && pairs < kSpillPairs));
+    const int pairs = streams_ * c_.heads, chunks = attn_chunks();
+    return dim_ <= 128 && chunks > 1 &&
+           (pairs < kSplitPairs || (pairs > kCuPairs && pairs < kSpillPairs && chunks > 2));
   }
   int column_tiles(int cols) const;
   bool folds_norm(int cols) const;

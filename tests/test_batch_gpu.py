@@ -163,7 +163,7 @@ def test_projection_shapes_equal_a_batch_of_one(weights, mixed, width, ffn, stre
     (68, 4, 130, 64, 133, True),    # the second piece of four elements
     (160, 2, 140, 3, 145, False),   # the wide form
     (32, 2, 1040, 130, 1050, False),  # nine chunks: more than a merge of a split window reads at once
-    # 320 pairs: walked (between 256 and 320 they are split, as below 192)
+    # 320 pairs: walked (three chunks or more of 257 to 319 pairs are split, as below 192)
     (64, 4, 129, 80, 135, False),
     (48, 4, 300, 80, 310, True),
     (128, 2, 200, 160, 210, False),
