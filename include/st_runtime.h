@@ -238,8 +238,8 @@ int st_batch_create(const st_config* config, int32_t mixed, const st_tensor* ten
  * single-stream step on its own share of the CUs (workgroups [s*per, (s+1)*per), per = the
  * CU count / streams, a multiple of 8 when at least 8), with its own state and the weights
  * shared. Each stream's scores and state are bit-identical to a single-stream runtime's (FUSED)
- * fed the same events. For small batches, which the phase-kernel graph above leaves
- * launch-bound. streams: 1..32. Every st_batch_* call below applies. */
+ * fed the same events, for which it is meant: the phase-kernel graph above is as fast at
+ * one stream and faster from four on. streams: 1..32. Every st_batch_* call below applies. */
 int st_batch_create_resident(const st_config* config, int32_t mixed, const st_tensor* tensors, size_t tensor_count,
                              int32_t streams, int32_t weight_dtype, st_batch** out);
 void st_batch_destroy(st_batch* batch);

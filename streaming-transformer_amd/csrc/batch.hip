@@ -135,13 +135,13 @@ int Batch::column_tiles(int cols) const {
 // Mixed mode: whether a projection of `cols` column tiles folds its norm. Folded, it saves the norm's
 // kernel and converts its X rows again in each group of column tiles; behind the norm's kernel it
 // takes X in FP16, four batch tiles to a workgroup. So it folds where there are no four tiles, else up
-// to kFoldWork values converted: rows x K x groups. us per layer of the fold against the norm's kernel,
+// to a line of values converted, rows x K x groups. us per layer of the fold against the norm's kernel,
 // swept over widths 256 to 1024, ffn 256 to 4096 and 1 to 256 streams: up to 32 streams always
-// less (-1.1 to -2.6). From 64 on, gate/up at 4.2 M -3.9 to -1.3, 8.4 M -0.6 to -0.1, 12.6 M -0.3 to
+// less (-1.1 to -2.6). From 64 on, gate/up at 4.2 M -3.9 to -1.3, 8.4 M -1.0 to -0.1, 12.6 M -0.3 to
 // +1.1, 16.8 M +2.8 and +3.4; QKV at 6.3 M -1.4 and -1.2, 9.4 M -0.1 to +0.4, 12.6 M -0.1 and +0.3. Odd
 // column tile counts, whose four-tile shape shares X with no second column tile: 11.3 M -0.8, 12.3 M
-// +0.6, 14.2 M +0.3, 16.7 M +2.1. (One width, 528, whose groups fall on the XCDs unevenly, loses 1 us at
-// 4.3 M.)
+// +0.6, 14.2 M +0.3, 16.7 M +2.1. (One width, 528, with its 33 groups of gate/up, loses 1 us at 4.3 M
+// from 128 streams on.)
 bool Batch::folds_norm(int cols) const {
   const size_t line = (size_t)(cols % 2 ? 12 : 8) << 20;
   return streams_p_ % (4 * kBatchTile) != 0 ||

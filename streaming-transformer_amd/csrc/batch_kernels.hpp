@@ -210,7 +210,7 @@ __device__ __forceinline__ void pin4(u32x2_t& v) { asm volatile("" : "+v"(v)); }
 // the MFMAs: the kernels that write x also write its squares summed over four columns
 // (kSquares), and each wave adds those of its slice while its first K blocks are in flight. This
 // saves the two norm kernels of a layer (about 2.5 us each) where the conversions that every
-// column tile's workgroup then repeats cost less (Batch::launch_sequence).
+// column tile's workgroup then repeats cost less (Batch::folds_norm).
 //
 // Everything a kernel needs before its first load comes in the kernel arguments (the first 16
 // dwords are preloaded into SGPRs). What only the epilogue needs (the residual, the RoPE table,
