@@ -147,8 +147,9 @@ __device__ __forceinline__ void split3(const float (&x)[8], unsigned (&ph)[4], u
 // fragments of block j as soon as block j's MFMAs are issued, so R blocks are in flight while one
 // computes. The host picks R = 4 for workgroups of at most two tiles when the slice holds a
 // multiple of 4 blocks (it always holds an even number), else 2.
-// Three things hold the schedule: an empty asm after each prefetch (the compiler would otherwise
-// see that the loads only feed the next round and move them next to their use); `pin`, which
+// Three things hold the schedule: an empty asm after each block's loads (the compiler would otherwise
+// see that a prefetch only feeds the next round and move it next to its use, and group the first
+// blocks' loads by operand, so that the first block waits for the last one's); `pin`, which
 // passes a fragment's registers through an asm right before its MFMAs (the compiler would
 // otherwise hoist the operand arithmetic of every fragment to the top of the round, which waits
 // for all loads in flight); and that the fragments are whole 4-register vectors in the pins too
@@ -162,8 +163,10 @@ __device__ __forceinline__ void k_ring(int k0, int slice, Load&& load, Pin&& pin
   const int nb = slice / KB;
   Frag f[R];
 #pragma unroll
-  for (int r = 0; r < R; r++) load(k0 + r * KB, f[r]);
-  asm volatile("" ::: "memory");
+  for (int r = 0; r < R; r++) {
+    load(k0 + r * KB, f[r]);
+    asm volatile("" ::: "memory");
+  }
   early();
   int j = 0;
   for (; j + R < nb; j += R) {
