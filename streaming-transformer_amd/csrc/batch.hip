@@ -140,12 +140,13 @@ int Batch::column_tiles(int cols) const {
 // less (-1.1 to -2.6). From 64 on, gate/up at 4.2 M -3.9 to -1.3, 8.4 M -1.0 to -0.1, 12.6 M -0.3 to
 // +1.1, 16.8 M +2.8 and +3.4; QKV at 6.3 M -1.4 and -1.2, 9.4 M -0.1 to +0.4, 12.6 M -0.1 and +0.3. Odd
 // column tile counts, whose four-tile shape shares X with no second column tile: 11.3 M -0.8, 12.3 M
-// +0.6, 14.2 M +0.3, 16.7 M +2.1. (One width, 528, with its 33 groups of gate/up, loses 1 us at 4.3 M
-// from 128 streams on.)
+// +0.6, 14.2 M +0.3, 16.7 M +2.1. Odd numbers of groups of four tiles lose sooner at the wider K:
+// 3.5 M and 3.9 M -1.6, 4.3 M to 5.9 M at 128 rows +0.7 to +2.0, 6.5 M +0.4 to +0.9 (at K = 512 still
+// -1.2 at 4.3 M, -1.1 at 4.9 M).
 bool Batch::folds_norm(int cols) const {
-  const size_t line = (size_t)(cols % 2 ? 12 : 8) << 20;
-  return streams_p_ % (4 * kBatchTile) != 0 ||
-         (size_t)streams_p_ * args_.width_p * (cols / column_tiles(cols)) <= line;
+  const int ct = column_tiles(cols), groups = cols / ct;
+  const size_t line = (size_t)(cols % 2 ? 12 : ct == 4 && groups % 2 && args_.width_p > 512 ? 4 : 8) << 20;
+  return streams_p_ % (4 * kBatchTile) != 0 || (size_t)streams_p_ * args_.width_p * groups <= line;
 }
 
 // One projection. Every workgroup shape computes the same fixed slice tree, so the choice changes
