@@ -84,7 +84,7 @@ ResidentBatch::ResidentBatch(const st_config& config, bool mixed, const st_tenso
   HIP_CHECK(hipMemcpy(stream_args_.ptr, all.data(), all.size() * sizeof(StepArgs), hipMemcpyHostToDevice));
   const size_t in_bytes = (size_t)streams * fp_ * 4;
   in_.alloc(in_bytes);
-  HIP_CHECK(hipMemset(in_.ptr, 0, in_bytes));
+  HIP_CHECK(hipMemsetAsync(in_.ptr, 0, in_bytes, stream_));  // before the first step's events, on their stream
   out_.alloc((size_t)streams * 8);
   host_in_.alloc(in_bytes);
   std::memset(host_in_.ptr, 0, in_bytes);

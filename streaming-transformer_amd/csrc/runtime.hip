@@ -522,7 +522,10 @@ __global__ __launch_bounds__(kThreads) void coresidency_kernel(unsigned* arrived
 bool Runtime::coresident(int grid) {
   DeviceBuffer words;
   words.alloc(256);
-  HIP_CHECK(hipMemset(words.ptr, 0, 256));
+  // On the launch's own stream: hipMemset runs on the null stream, which a non-blocking stream does
+  // not wait for, and returns before device memory is cleared. Cleared late, the count of arrivals
+  // was lost and the probe failed on an idle chip.
+  HIP_CHECK(hipMemsetAsync(words.ptr, 0, 256, stream_));
   unsigned* w = reinterpret_cast<unsigned*>(words.ptr);
   const unsigned long long ticks = (unsigned long long)wall_khz_ * 50ull;  // 50 ms
   hipLaunchKernelGGL(coresidency_kernel, dim3(grid), dim3(kThreads), 0, stream_, w, (unsigned)grid, ticks, w + 32);
@@ -1568,8 +1571,6 @@ std::string transport_bench(const std::string& mode, uint64_t count, bool backof
   d_out.alloc(128);
   d_ticks.alloc(count * 8);
   d_errors.alloc(4);
-  HIP_CHECK(hipMemset(d_errors.ptr, 0, 4));
-  HIP_CHECK(hipMemset(d_ticks.ptr, 0, count * 8));
   hipStream_t stream;
   HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   struct StreamGuard {
@@ -1583,6 +1584,8 @@ std::string transport_bench(const std::string& mode, uint64_t count, bool backof
       (void)hipStreamDestroy(s);
     }
   } guard{stream};
+  HIP_CHECK(hipMemsetAsync(d_errors.ptr, 0, 4, stream));
+  HIP_CHECK(hipMemsetAsync(d_ticks.ptr, 0, count * 8, stream));
   if (mode == "empty-graph") {
     HIP_CHECK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(transport_empty_kernel, dim3(1), dim3(1), 0, stream);
